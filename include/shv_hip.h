@@ -125,7 +125,7 @@ void shv_hip_host_free(void* p);
  * forward on buffers already resident in HBM, without the scheduler or any host copy.
  * Device pointers only; `stream` is a hipStream_t (NULL = the model's compute stream).  Not thread-safe against
  * the model's own worker: call them only while no job is queued or running on `m`.  The calls are asynchronous and
- * share the model's activation buffers (and, in fp32, its small-GEMM workspace): calls on one model must run one
+ * share the model's activation buffers: calls on one model must run one
  * after another on the device -- issue them on one stream, or synchronise between streams.
  */
 /* d_frames: n_clips*20 crops in device memory; d_logits: n_clips fp32 in device memory.  n_clips <= limits. */
@@ -151,7 +151,7 @@ int shv_hip_set_dump_dir(shv_hip_model* m, const char* dir);
 /* Pointwise-conv GEMM microbench.  No counterpart in shv_cuda.h: the reference benches its GEMM from a C++ tool
  * (bench/gpu_gemm_bench.cu:27-116: engine GEMM on the model's 1x1 shapes, and a bitwise check that every kernel
  * variant gives the same outputs).  C[m][n] = act(A[m][k] . W[n][k]^T + bias[n]) in the arithmetic of `mode`
- * ("fp32": fp32 matrix cores, or the CPU engine's VALU order; "fp16" / "bf16": split-operand MFMA), fp32 A, W, bias and C in
+ * ("fp32": the CPU engine's operation order; "fp16" / "bf16": split-operand MFMA), fp32 A, W, bias and C in
  * device memory, row-major with leading dimensions k (A, W) and n (C).  act: the reference's codes
  * (engine/cuda/common.cuh:69): 0 none, 1 ReLU, 2 hardswish, 3 SiLU, 4 hardsigmoid.  d_bias may be NULL.
  * create repacks W on the device (synchronising `stream`); NULL + last_error on failure (fp16 / bf16 need k % 8 == 0).

@@ -233,7 +233,7 @@ private:
     }
 
     void gemm(const char* role, const GemmArgs& p, const DevW& w, hipStream_t s) {
-        GemmRunner<G>{*this, nullptr, 0, false}.gemm(role, p, w, s);
+        GemmRunner<G>{*this, false}.gemm(role, p, w, s);
     }
 
     // PCM windows [n] (window w at pcm + w * stride) -> tokens [n][125][384] at `tokens`, in chunks of front_chunk_

@@ -187,7 +187,6 @@ public:
         const Slot& sl = slots_.at(size_t(slot));
         const int Bb = window_bucket(B);
         run_graph(GraphKey{1, sl.d_tokptr, sl.d_logits, Bb}, s, [&](hipStream_t q) {
-            ws_on_ = true;   // one pass on q
             run_classify(sl.d_tokptr, Bb, sl.d_logits, q, 0);
         });
     }
@@ -217,13 +216,12 @@ public:
         if (n <= 0) return;
         if (n > cfg_.max_windows) throw std::runtime_error("classify: too many windows");
         run_graph(GraphKey{5, d_tokens, d_logits, n}, s, [&](hipStream_t q) {
-            ws_on_ = true;   // one pass on q
             WindowInput in;
             in.tokens = d_tokens;
             in.ldw = (long long)kFrames * kTokenFloats;
             in.pos = pos_;
             in.readout = readout_;
-            seq_->run(in, n, d_logits, q, *this, dump_dir_, 0, cur_ws(), ws_floats_);
+            seq_->run(in, n, d_logits, q, *this, dump_dir_);
         });
     }
 
@@ -374,14 +372,6 @@ private:
     // the scheduler's 32-clip batches (the reference's default options) then run as two (128 clips end to end from
     // pinned memory 4,977 -> 5,286 clips/s); 8 branches of 16 clips at batch 128 measured 20.7 vs 18.4 ms.
     static constexpr int kBranches = 4, kBranchClips = 16;
-    // Exact tier: the workspace of the small-M GEMMs' K-block sums (gemm_f32 with ws).  One per engine, so only a
-    // pass that runs alone on its stream hands it out: ws_on_ is set by each pass before it queues its kernels
-    // (false for branched passes, whose branches run at once).  32 MB covers every small-M GEMM of one clip.
-    static constexpr long long kWsFloats = 8ll << 20;
-    float* ws_ = nullptr;
-    long long ws_floats_ = 0;
-    bool ws_on_ = false;
-    float* cur_ws() const { return ws_on_ ? ws_ : nullptr; }
     hipStream_t bstream_[kBranches] = {};
     hipEvent_t fork_ = nullptr, join_[kBranches] = {};
     float* tok_direct_ = nullptr;
@@ -414,10 +404,6 @@ private:
         acts_.se_pool = amem_.make<float>(Fm * kCnnOut);
         acts_.se_hid = amem_.make<float>(Fm * 256);
         acts_.se_scale = amem_.make<float>(Fm * kCnnOut);
-        if constexpr (kF32) {
-            ws_floats_ = kWsFloats;
-            ws_ = amem_.make<float>(size_t(ws_floats_));
-        }
         // direct path: the engine's own token buffer and the window -> frame table of a plain predict
         const size_t Fd = std::min(Fm, Bm * kFrames);
         tok_direct_ = amem_.make<float>(Fd * kTokenFloats);
@@ -478,10 +464,10 @@ private:
 
     // GEMM in this engine's flavour, and the exact fp32 VALU kernel for the fp32-only layers
     void gemm(const char* role, const GemmArgs& p, const DevW& w, hipStream_t s) {
-        GemmRunner<G>{*this, cur_ws(), ws_floats_, cpu_order_}.gemm(role, p, w, s);
+        GemmRunner<G>{*this, cpu_order_}.gemm(role, p, w, s);
     }
     void gemm32(const char* role, const GemmArgs& p, hipStream_t s) {
-        GemmRunner<G>{*this, cur_ws(), ws_floats_, cpu_order_}.gemm32(role, p, s);
+        GemmRunner<G>{*this, cpu_order_}.gemm32(role, p, s);
     }
 
     // ---------------------------------------------------------------- CNN
@@ -502,7 +488,6 @@ private:
                           hipStream_t q) {
         const int nb = dump_dir_.empty() ? std::max(1, std::min(kBranches, n / kBranchClips)) : 1;
         const bool fork = nb > 1 && !profiling();
-        ws_on_ = nb == 1;
         const int sg = std::min(nb, kSeqGroup);
         const auto clip = [&](int b) { return int((long long)n * b / nb); };
         if (fork) SHV_HIP_CHECK(hipEventRecord(fork_, q));
@@ -531,7 +516,6 @@ private:
     void encode_branched(const uint8_t* frames, int F, float* tokens, hipStream_t q) {
         const int nb = dump_dir_.empty() ? std::max(1, std::min(kBranches, F / (kBranchClips * kFrames))) : 1;
         const bool fork = nb > 1 && !profiling();
-        ws_on_ = nb == 1;
         if (fork) SHV_HIP_CHECK(hipEventRecord(fork_, q));
         for (int b = 0; b < nb; ++b) {
             const int f0 = int((long long)F * b / nb), f1 = int((long long)F * (b + 1) / nb);
@@ -738,7 +722,7 @@ private:
         in.frame_tokens = tokptr;
         in.pos = pos_;
         in.readout = readout_;
-        seq_->run(in, B, logits, s, *this, dump_dir_, w0, cur_ws(), ws_floats_);
+        seq_->run(in, B, logits, s, *this, dump_dir_, w0);
     }
 };
 

@@ -14,6 +14,7 @@
 //   A and W tiles are staged through LDS (A split once per workgroup), the next K step prefetched into registers;
 //   K advances in steps of 32 in increasing order; a K tail is zero-filled, never split across waves.
 #include "dev_common.hpp"
+#include "gemm_epi.hpp"
 #include "kernels.hpp"
 #include "mfma.hpp"
 
@@ -25,44 +26,6 @@
 
 namespace shv {
 namespace {
-
-// ------------------------------------------------------------------------------------------------ epilogue
-// out = act(v * wscale + bias) (+ residual: res 1 R + v, res 2 R + v / sqrt(2), res 3 R + 0.70710678f * v).  wscale
-// is a power of two (1 unless the weight was stored pre-scaled), so v * wscale is exact.
-__device__ __forceinline__ float epi_value(const GemmArgs& p, float v, float b, float res) {
-    v = v * p.wscale;
-    if (p.bias) v = v + b;
-    v = apply_act(v, p.act);
-    if (p.res == 3) v = res + 0.7071067811865475244f * v;
-    else if (p.res) v = p.res == 2 ? res + v / 1.41421356237309515f : res + v;
-    return v;
-}
-// Epilogue of the 4 x J outputs one thread holds (rows row(i), columns col(j)).  Every bias and residual operand is
-// loaded (at clamped, valid addresses) before the first store: C may alias R or the bias as far as the compiler
-// knows, so a load written after a store would wait for it, one memory round trip per output.
-template <int J, class Row, class Col, class Val>
-__device__ __forceinline__ void epi_block(const GemmArgs& p, Row row, Col col, Val val) {
-    float bv[J], rv[4][J];
-#pragma unroll
-    for (int j = 0; j < J; ++j) bv[j] = p.bias ? p.bias[min(col(j), p.N - 1)] : 0.0f;
-    if (p.res) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < J; ++j)
-                rv[i][j] = p.R[min(row(i), (long long)p.M - 1) * p.ldr + min(col(j), p.N - 1)];
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const long long m = row(i);
-        if (m >= p.M) continue;
-#pragma unroll
-        for (int j = 0; j < J; ++j) {
-            const int n = col(j);
-            if (n < p.N) p.C[m * p.ldc + n] = epi_value(p, val(i, j), bv[j], p.res ? rv[i][j] : 0.0f);
-        }
-    }
-}
 
 // SwiGLU of the MFMA tiers from the gate and up sums
 __device__ __forceinline__ float swiglu_value(const GemmArgs& p, float gate, float up) {
@@ -537,129 +500,6 @@ __global__ void __launch_bounds__(256) gemm_f32_cols_kernel(GemmArgs p) {
         const int row = i / NC, j = i % NC;
         if (m0 + row < p.M && n0 + j < p.N) p.C[(m0 + row) * p.ldc + n0 + j] = ct[row * CS + j];
     }
-}
-
-// ------------------------------------------------------------------------------------------------ fp32 MFMA
-// The fp32 tier's all-row sequence GEMMs on the matrix cores: v_mfma_f32_16x16x4_f32 takes fp32 operands, forms
-// fp32 products and accumulates in fp32 (no reduced-precision operand type).  Fragment layout, lane l = 16 g + r:
-// A holds row r at k slot g, B column r at k slot g, C column r at rows 4 g .. 4 g + 3.
-// A workgroup of four waves owns MT x NT blocks of 16 x 16 and splits K between its waves: K runs in steps of 16,
-// and wave w takes steps w, w + 4, w + 8, ... in increasing order.  Per step, lane (g, r) loads A[row][k0 + 4 g ..
-// + 3] and W[column][k0 + 4 g .. + 3] as one float4 each straight from memory (no LDS staging), and MFMA kk (0..3)
-// takes k = k0 + 4 g + kk in slot g, into the wave's accumulator from +0.  The four partial sums are then added as
-// (w0 + w1) + (w2 + w3) through LDS and wave 0 runs the epilogue.  Every output therefore receives the same
-// operations whatever MT, NT, D, M or the other rows: results are bitwise independent of the tiling and of the
-// batch.  Each wave keeps D of its steps' operands in flight (the 321-row GEMMs of one clip are bound by load
-// latency, not by the matrix cores).  K, lda, ldw (and ld_scale) are multiples of 4; a K tail loads clamped
-// addresses and zeros.
-template <int MT, int NT, int D, bool SCALE>
-__global__ void __launch_bounds__(256) gemm_f32_mfma_kernel(GemmArgs p) {
-    __shared__ f32x4 part[3][MT][NT][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int g = lane >> 4, r = lane & 15;
-    const long long mbase = (long long)blockIdx.x * (MT * 16);
-    const int nbase = blockIdx.y * (NT * 16);
-    const float* W = static_cast<const float*>(p.W);
-    const float* arow[MT];
-    const float* srow[MT];
-    bool alive[MT];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-        const long long m = mbase + mt * 16 + r;
-        alive[mt] = m < p.M;
-        const long long mc = alive[mt] ? m : p.M - 1;
-        arow[mt] = p.A + mc * p.lda + 4 * g;
-        srow[mt] = SCALE ? p.scale + (mc / p.scale_rows) * p.ld_scale + 4 * g : nullptr;
-    }
-    const float* wrow[NT];
-    bool wlive[NT];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-        const int n = nbase + nt * 16 + r;
-        wlive[nt] = n < p.N;
-        wrow[nt] = W + (long long)(wlive[nt] ? n : p.N - 1) * p.ldw + 4 * g;
-    }
-    const auto load = [&](int k0, float4 (&a)[MT], float4 (&w)[NT]) {
-        const bool kin = k0 + 4 * g < p.K;
-        const int kc = kin ? k0 : p.K - 4 - 4 * g;   // clamped so that the float4 stays inside the row
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-            float4 v = *reinterpret_cast<const float4*>(arow[mt] + kc);
-            if (SCALE) {
-                const float4 sc = *reinterpret_cast<const float4*>(srow[mt] + kc);
-                v = make_float4(sc.x * v.x, sc.y * v.y, sc.z * v.z, sc.w * v.w);
-            }
-            a[mt] = (kin && alive[mt]) ? v : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        }
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            const float4 v = *reinterpret_cast<const float4*>(wrow[nt] + kc);
-            w[nt] = (kin && wlive[nt]) ? v : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        }
-    };
-    f32x4 acc[MT][NT];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    // this wave's steps wave + 4 i; step i sits in ring slot i % D and is reloaded with step i + D once consumed
-    const int nsteps = (p.K + 15) / 16, mine = (nsteps - wave + 3) / 4;
-    float4 a[D][MT], w[D][NT];
-#pragma unroll
-    for (int d = 0; d < D; ++d)
-        if (d < mine) load(16 * (wave + 4 * d), a[d], w[d]);
-    for (int i0 = 0; i0 < mine; i0 += D) {
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-            const int i = i0 + d;
-            if (i >= mine) break;
-#pragma unroll
-            for (int kk = 0; kk < 4; ++kk)
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                    for (int nt = 0; nt < NT; ++nt) {
-                        const float av = kk == 0 ? a[d][mt].x : kk == 1 ? a[d][mt].y : kk == 2 ? a[d][mt].z : a[d][mt].w;
-                        const float wv = kk == 0 ? w[d][nt].x : kk == 1 ? w[d][nt].y : kk == 2 ? w[d][nt].z : w[d][nt].w;
-                        acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, wv, acc[mt][nt], 0, 0, 0);
-                    }
-            if (i + D < mine) load(16 * (wave + 4 * (i + D)), a[d], w[d]);
-        }
-    }
-    if (wave) {
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) part[wave - 1][mt][nt][lane] = acc[mt][nt];
-    }
-    __syncthreads();
-    if (wave) return;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-            acc[mt][nt] = (acc[mt][nt] + part[0][mt][nt][lane]) + (part[1][mt][nt][lane] + part[2][mt][nt][lane]);
-    // lane holds C[mbase + mt * 16 + 4 g + i][nbase + nt * 16 + r]
-    if (p.swiglu) {   // weight rows in 16-row panels alternating gate / up: NT even, nbase a multiple of 32
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const long long m = mbase + mt * 16 + 4 * g + i;
-                if (m >= p.M) continue;
-#pragma unroll
-                for (int nt = 0; nt + 1 < NT; nt += 2) {
-                    const int panel = nbase / 16 + nt;
-                    if ((panel + 1) * 16 <= p.N)
-                        p.C[m * p.ldc + (panel / 2) * 16 + r] = silu(acc[mt][nt][i]) * acc[mt][nt + 1][i];
-                }
-            }
-        return;
-    }
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-        epi_block<NT>(p, [&](int i) { return mbase + mt * 16 + 4 * g + i; }, [&](int j) { return nbase + j * 16 + r; },
-                      [&](int i, int j) { return acc[mt][j][i]; });
 }
 
 // Small M (<= 256 rows, e.g. the windows' last SISA rows): the same per-element arithmetic as gemm_f32_kernel -- K blocks
@@ -2113,7 +1953,11 @@ bool narrow_f32_shape(const GemmArgs& p, bool launch, hipStream_t s) {
         }
     return false;
 }
-bool use_narrow_f32(const GemmArgs& p) { return p.M >= 4096 && narrow_f32_shape(p, false, nullptr); }
+// Of these only block 1's 16 -> 16, all loads and stores, is faster here than on the matrix cores (4,608,000 rows: 119
+// against 142 us; 16 -> 64 569 against 382, 64 -> 24 267 against 84, 120 -> 40 145 against 49).
+bool use_narrow_f32(const GemmArgs& p) {
+    return p.M >= 4096 && p.K == 16 && p.N == 16 && narrow_f32_shape(p, false, nullptr);
+}
 bool cols_f32_ok(const GemmArgs& p) {
     const auto al16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
     return !p.swiglu && p.K % 4 == 0 && p.K <= COLS_KMAX && p.lda % 4 == 0 && p.ldw % 4 == 0 && p.lda >= p.K &&
@@ -2135,51 +1979,24 @@ void launch_narrow_f32(const GemmArgs& p, hipStream_t s) {
         throw std::runtime_error("gemm_f32: no narrow kernel for K=" + std::to_string(p.K) + " N=" + std::to_string(p.N) +
                                  " with these leading dimensions / alignments");
 }
-// The exact-tier kernel for M above the GEMV range: K blocks in parallel when the tiled grid would not give every
-// CU a workgroup and the workspace holds the block sums (measured with one clip: blocks 13-15 SE projects, 57
-// tiles, and the 321-row sequence GEMMs ran 45-200 us on the tiled kernel)
-bool use_kblock_f32(const GemmArgs& p) {
-    const long long nkb = cdiv(p.K, F32_BK), tiles = (long long)cdiv(p.M, F32_BM) * cdiv(p.N, F32_BN);
-    return p.ws && nkb >= 2 && tiles < 256 && nkb * p.M * p.N <= p.ws_floats;
-}
-}  // namespace
-
-namespace {
-struct F32MfmaTile {
-    int mt, nt;
-};
-// Tiles of the fp32 matrix-core GEMM by shape (every choice gives the same per-output operations): 32 x 64 per
-// workgroup while that grid gives every CU eight workgroups, 16 x 32 below (one clip's 321-row GEMMs: 252 to 1,533
-// workgroups instead of 66 to 407).
-F32MfmaTile plan_f32_mfma(const GemmArgs& p) {
-    if ((long long)cdiv(p.M, 32) * cdiv(p.N, 64) >= 2048) return {2, 4};
-    return {1, 2};
-}
-template <int MT, int NT> void launch_f32_mfma(const GemmArgs& p, hipStream_t s) {
-    constexpr int D = MT * NT >= 8 ? 2 : 4;   // K steps in flight per wave: deeper for the small tiles
-    const dim3 grid(cdiv(p.M, MT * 16), cdiv(p.N, NT * 16));
-    if (p.scale) hipLaunchKernelGGL((gemm_f32_mfma_kernel<MT, NT, D, true>), grid, dim3(256), 0, s, p);
-    else hipLaunchKernelGGL((gemm_f32_mfma_kernel<MT, NT, D, false>), grid, dim3(256), 0, s, p);
+// Few rows stay on the GEMV, which reads W once whatever its alignment (one row: 6.1-6.2 us against 7.0-7.2 of the
+// matrix-core kernels; 20 rows 7.3-9.5 against 6.3-7.4, 128 rows 22-56 against 7-9); without the matrix cores' alignment
+// it serves every M it takes.
+bool use_gemv_f32(const GemmArgs& p) {
+    return p.M <= (gemm_f32_mc_ok(p) ? 4 : GV_MAXM) && cdiv(p.K, F32_BK) <= 32;
 }
 }  // namespace
 
 void gemm_f32_mfma(const GemmArgs& p, hipStream_t s) {
     check_args(p, false);
-    const auto al16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
-    if (p.K % 4 || p.lda % 4 || p.ldw % 4 || !al16(p.A) || !al16(p.W) ||
-        (p.scale && (p.ld_scale % 4 || !al16(p.scale))))
+    if (!gemm_f32_mc_ok(p))
         throw std::runtime_error("gemm_f32_mfma: K, lda, ldw, ld_scale must be multiples of 4 and A, W, scale "
                                  "16-byte aligned (K=" + std::to_string(p.K) + ")");
     if (p.swiglu && p.N % 32) throw std::runtime_error("gemm_f32_mfma: swiglu needs N % 32 == 0");
-    const F32MfmaTile t = plan_f32_mfma(p);
-    if (t.mt == 2) launch_f32_mfma<2, 4>(p, s);
-    else launch_f32_mfma<1, 2>(p, s);
+    gemm_f32_mc(p, p.swiglu ? 2 : 0, s);
 }
 
-std::string gemm_f32_mfma_kernel_name(const GemmArgs& p) {
-    const F32MfmaTile t = plan_f32_mfma(p);
-    return "gemm_f32_mfma_kernel<" + std::to_string(t.mt) + "," + std::to_string(t.nt) + ">";
-}
+std::string gemm_f32_mfma_kernel_name(const GemmArgs& p) { return gemm_f32_mc_kernel(p, p.swiglu ? 2 : 0); }
 
 void gemm_f32(const GemmArgs& p, hipStream_t s) { gemm_f32_variant(p, s, 0); }
 
@@ -2187,9 +2004,9 @@ void gemm_f32_variant(const GemmArgs& p, hipStream_t s, int variant) {
     check_args(p, false);
     switch (variant) {
     case 0:
-        if (p.M <= GV_MAXM && cdiv(p.K, F32_BK) <= 32) launch_gemv_f32(p, s);
+        if (use_gemv_f32(p)) launch_gemv_f32(p, s);
         else if (use_narrow_f32(p)) launch_narrow_f32(p, s);
-        else if (use_kblock_f32(p)) launch_kblock_f32(p, s);
+        else if (gemm_f32_mc_ok(p)) gemm_f32_mc(p, p.swiglu ? 1 : 0, s);
         else launch_tiled_f32(p, s);
         return;
     case 1: launch_gemv_f32(p, s); return;
@@ -2202,10 +2019,10 @@ void gemm_f32_variant(const GemmArgs& p, hipStream_t s, int variant) {
 }
 
 std::string gemm_f32_kernel(const GemmArgs& p) {
-    if (p.M <= GV_MAXM && cdiv(p.K, F32_BK) <= 32) return "gemv_f32_kernel";
+    if (use_gemv_f32(p)) return "gemv_f32_kernel";
     if (use_narrow_f32(p)) return "gemm_f32_narrow_kernel<" + std::to_string(p.K) + "," + std::to_string(p.N) + ">";
-    if (v4_f32_ok(p)) return use_kblock_f32(p) ? "gemm_f32_v4_kernel<part>" : "gemm_f32_v4_kernel";
-    return use_kblock_f32(p) ? "gemm_f32_kblock_kernel" : "gemm_f32_kernel";
+    if (gemm_f32_mc_ok(p)) return gemm_f32_mc_kernel(p, p.swiglu ? 1 : 0);
+    return v4_f32_ok(p) ? "gemm_f32_v4_kernel" : "gemm_f32_kernel";
 }
 
 template <typename T> std::string gemm_mfma_kernel(const GemmArgs& p) {

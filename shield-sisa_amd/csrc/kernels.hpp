@@ -41,20 +41,22 @@ struct GemmArgs {
     // kstride >= rows * 32: each 16 x 32 fragment block 1 KB contiguous) are read by the small-M, LDS-staged and
     // direct-to-LDS kernels (the sequence GEMMs); the other kernels take the default only.
     long long wkstride = 32, akstride = 32, ckstride = 32;
-    // Exact tier: device workspace of ws_floats floats the GEMM may use for its K-block sums when M is small (the
-    // caller guarantees no other launch uses it meanwhile); null: never.
+    // The VALU K-block kernel's device workspace of ws_floats floats (gemm_f32_variant 3).
     float* ws = nullptr; long long ws_floats = 0;
 };
 
-// fp32 tier: VALU GEMM, each output accumulated in K blocks of 64 (fma chain from +0 per block, block sums added
-// in order) exactly as the reference CPU engine (engine/model/isa_impl.hpp:188-317).
+// fp32 tier: each output accumulated in K blocks of 64 (fma chain from +0 per block, block sums added in order) exactly
+// as the reference CPU engine (engine/model/isa_impl.hpp:188-317), on the fp32 matrix cores where K, lda, ldw and the
+// scale rows are multiples of 4 and 16-byte aligned, else on the VALU kernels (the same sequence, bitwise equal).
 void gemm_f32(const GemmArgs& p, hipStream_t s);
-// fp32 tier, all-row sequence GEMMs: v_mfma_f32_16x16x4_f32 (fp32 operands, products and accumulation).  Per
-// output, K in steps of 16 dealt round robin over four partial sums (each from +0, in increasing k, four MFMAs per
-// step), added as (p0 + p1) + (p2 + p3): the same for every tile, M and batch (row independence).  SwiGLU weights in
-// 16-row gate / up panels (repack perm 2).
+// The same with SwiGLU weights in 16-row gate / up panels (repack perm 2); matrix cores only.
 void gemm_f32_mfma(const GemmArgs& p, hipStream_t s);
 std::string gemm_f32_mfma_kernel_name(const GemmArgs& p);
+// The matrix-core kernels behind both (gemm_f32.hip): whether they take these arguments (checked by the callers above),
+// the launch, its kernel's name.  swiglu: 0 none, 1 adjacent gate / up columns, 2 16-column panels.
+bool gemm_f32_mc_ok(const GemmArgs& p);
+void gemm_f32_mc(const GemmArgs& p, int swiglu, hipStream_t s);
+std::string gemm_f32_mc_kernel(const GemmArgs& p, int swiglu);
 // fp16 / bf16 tiers: MFMA 16x16x32 on split operands (fp16 2 parts / 3 products, bf16 3 parts / 6 products) with
 // fp32 accumulation, K consumed in 32-wide steps in increasing order (no split-K): a row's outputs do not depend
 // on M, the tile, or other rows.

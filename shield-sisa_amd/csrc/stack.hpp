@@ -20,8 +20,8 @@ namespace shv {
 
 inline void check_launch() { SHV_HIP_CHECK(hipGetLastError()); }
 
-// G selects how GEMM operands reach the multipliers: float = fp32 (matrix cores, or the reference's VALU order),
-// f16 / bf16 = split-operand MFMA
+// G selects how GEMM operands reach the multipliers: float = fp32 in the reference's K-block order (cpu_order: SwiGLU
+// weights as gate / up pairs instead of 16-row panels), f16 / bf16 = split-operand MFMA
 template <typename G> inline void gemm_t(const GemmArgs& p, hipStream_t s, bool cpu_order);
 template <> inline void gemm_t<float>(const GemmArgs& p, hipStream_t s, bool cpu_order) {
     if (cpu_order) gemm_f32(p, s);
@@ -183,9 +183,7 @@ template <typename U> void dump_f32(const std::string& dir, const char* name, co
 template <typename G> struct GemmRunner {
     static constexpr bool kF32 = std::is_same<G, float>::value;
     Profiler& pf;
-    float* ws = nullptr;   // the exact GEMM's small-M workspace (gemm_f32), null when the caller has none free
-    long long ws_floats = 0;
-    bool cpu_order = false;   // fp32 tier: the reference CPU order instead of the fp32 matrix cores
+    bool cpu_order = false;   // fp32 tier: SwiGLU weights in the VALU kernels' gate / up pairs
     std::string family(const char* role, const GemmArgs& p, bool f32) const {
         if (!pf.profiling()) return std::string();
         if constexpr (!kF32) {
@@ -197,10 +195,6 @@ template <typename G> struct GemmRunner {
     }
     // in this flavour's arithmetic; A is read pre-split where the producer wrote parts, else as fp32
     void gemm(const char* role, GemmArgs p, const DevW& w, hipStream_t s) const {
-        if constexpr (kF32) {
-            p.ws = ws;
-            p.ws_floats = ws_floats;
-        }
         p.W = w.w;
         p.wstride = w.stride;
         p.wscale = w.scale;
@@ -215,11 +209,8 @@ template <typename G> struct GemmRunner {
         pf.timed(family(role, p, false), bytes, s, [&] { gemm_t<G>(p, s, cpu_order); }, 2.0 * p.M * p.N * p.K);
         check_launch();
     }
-    // the exact fp32 VALU kernel (layers kept in fp32 in every tier)
-    void gemm32(const char* role, const GemmArgs& p0, hipStream_t s) const {
-        GemmArgs p = p0;
-        p.ws = ws;
-        p.ws_floats = ws_floats;
+    // in fp32 (layers kept in fp32 in every tier)
+    void gemm32(const char* role, const GemmArgs& p, hipStream_t s) const {
         pf.timed(family(role, p, true), gemm_bytes(p.M, p.N, p.K, 4, 4, p.swiglu ? 2 : 4, p.res ? 4 : 0), s,
                  [&] { gemm_f32(p, s); }, 2.0 * p.M * p.N * p.K);
         check_launch();
@@ -316,9 +307,9 @@ public:
     // B windows read from `in` -> logits[B], in windows [w0, w0 + B) of every buffer (disjoint window ranges can
     // run at once on different streams)
     void run(const WindowInput& in, int B, float* logits, hipStream_t s, Profiler& pf, const std::string& dump_dir,
-             int w0 = 0, float* ws = nullptr, long long ws_floats = 0) {
+             int w0 = 0) {
         const int T = spec_.T, M = B * T;
-        const GemmRunner<G> gr{pf, ws, ws_floats, cpu_order_};
+        const GemmRunner<G> gr{pf, cpu_order_};
         const size_t r0 = size_t(w0) * T;   // first row
         float *H = this->H_ + r0 * kD, *P = this->P_ + r0 * kGld, *Q = this->Q_ + r0 * kD,
               *K = this->K_ + r0 * kD, *V = this->V_ + r0 * kVD, *dec = this->dec_ + r0 * 8,

@@ -28,11 +28,11 @@ LIB = PKG / "lib"
 INCLUDE = PKG.parent / "include"
 
 NUMERIC_SOURCES = ["dev_common.hpp", "mfma.hpp", "kernels.hpp", "gemm_epi.hpp", "gemm.hip",
-                   "gemm_f32.hip", "cnn.hip", "fused.hip", "strip.hip", "seq.hip",
+                   "gemm_f32.hpp", "gemm_f32.hip", "cnn.hip", "expdw.hip", "fused.hip", "strip.hip", "seq.hip",
                    "engine.hpp", "engine.hip", "stack.hpp", "audio.hpp", "audio.hip", "afront.hip",
                    "host_model.hpp", "host_model.cpp"]
-DEVICE_SOURCES = ["gemm.hip", "gemm_f32.hip", "cnn.hip", "fused.hip", "strip.hip", "seq.hip", "engine.hip", "audio.hip", "afront.hip",
-                  "crop.hip"]
+DEVICE_SOURCES = ["gemm.hip", "gemm_f32.hip", "cnn.hip", "expdw.hip", "fused.hip", "strip.hip", "seq.hip", "engine.hip",
+                  "audio.hip", "afront.hip", "crop.hip"]
 HOST_SOURCES = ["host_model.cpp", "sched.cpp", "cert.cpp"]
 HIP_HOST_SOURCES = ["lanes.cpp"]          # host code that calls the HIP runtime
 API_SOURCE = "capi.cpp"                   # built twice: certified and experimental
@@ -50,7 +50,7 @@ DEVICE_FLAGS = ["--offload-arch=" + ARCH, "-Xclang", "-target-feature", "-Xclang
 # an asm operand, and an empty asm is counted as one wait state.  In these two files every asm operand is a loaded
 # value or a VALU result; tests/test_mfma_asm_hazard.py checks that on the built code objects (no inline-asm DPP
 # instruction reads a VGPR that an MFMA write can reach).
-VGPR_FORM_SOURCES = {"strip.hip", "gemm.hip", "gemm_f32.hip"}
+VGPR_FORM_SOURCES = {"strip.hip", "gemm.hip", "gemm_f32.hip", "expdw.hip"}
 VGPR_FORM_FLAGS = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 
 

@@ -149,7 +149,7 @@ private:
             return std::tie(kind, in, ldw, out, n) < std::tie(o.kind, o.in, o.ldw, o.out, o.n);
         }
     };
-    // the frontend runs over chunks of this many windows (its activations: about 49 MB per window)
+    // the frontend runs over chunks of this many windows (its activations: about 28 MB per window)
     static constexpr int kFrontChunk = 16;
     struct FrontBlock {
         int ci, hid, co, sf, st, T, F, To, Fo;
@@ -164,8 +164,8 @@ private:
     DevW proj_w_;
     int front_chunk_ = 0;
     // frontend activations for front_chunk_ windows: PCM staging (host calls), log-mel, block input / output
-    // ping-pong, pw1 output, depthwise output, pooled attention output
-    float *d_pcm_ = nullptr, *d_mel_ = nullptr, *d_x_[2] = {nullptr, nullptr}, *d_e_ = nullptr, *d_dwo_ = nullptr,
+    // ping-pong, depthwise output, pooled attention output
+    float *d_pcm_ = nullptr, *d_mel_ = nullptr, *d_x_[2] = {nullptr, nullptr}, *d_dwo_ = nullptr,
           *d_pool_ = nullptr;
 
     void need_frontend() const {
@@ -193,7 +193,7 @@ private:
         stem_scale_ = upl.up(F.stem_scale);
         stem_shift_ = upl.up(F.stem_shift);
         int T = kAudioMelFrames, Fq = kAudioMelBins;
-        size_t xmax = size_t(T) * Fq * 32, emax = 0, dmax = 0;
+        size_t xmax = size_t(T) * Fq * 32, dmax = 0;
         for (int i = 0; i < 8; ++i) {
             const AudioBlockHost& h = F.blocks[i];
             FrontBlock& b = fblk_[i];
@@ -209,7 +209,6 @@ private:
             b.dw_w = upl.up(h.dw_w);
             b.dw_scale = upl.up(h.dw_scale);
             b.dw_shift = upl.up(h.dw_shift);
-            emax = std::max(emax, size_t(T) * Fq * h.hid);
             dmax = std::max(dmax, size_t(b.To) * b.Fo * h.hid);
             xmax = std::max(xmax, size_t(b.To) * b.Fo * h.co);
             T = b.To;
@@ -226,7 +225,6 @@ private:
         d_mel_ = amem_.make<float>(c * kAudioMelFrames * kAudioMelBins);
         d_x_[0] = amem_.make<float>(c * xmax);
         d_x_[1] = amem_.make<float>(c * xmax);
-        d_e_ = amem_.make<float>(c * emax);
         d_dwo_ = amem_.make<float>(c * dmax);
         d_pool_ = amem_.make<float>(c * kAudioTokensPerWindow * kAudioCnnCh);
         has_frontend_ = true;
@@ -251,15 +249,12 @@ private:
             for (int i = 0; i < 8; ++i) {
                 const FrontBlock& k = fblk_[i];
                 const long long rows_in = (long long)b * k.T * k.F, rows_out = (long long)b * k.To * k.Fo;
-                GemmArgs p1;
-                p1.M = int(rows_in); p1.N = k.hid; p1.K = k.ci;
-                p1.A = d_x_[cur]; p1.lda = k.ci; p1.ldw = k.ci;
-                p1.bias = k.b1; p1.act = ACT_SILU;
-                p1.C = d_e_; p1.ldc = k.hid;
-                gemm("audio_pw1", p1, k.pw1, s);
-                timed("audio_dw", double(rows_in + rows_out) * k.hid * 4, s, [&] {
-                    launch_audio_dw(d_e_, d_dwo_, k.dw_w, k.dw_scale, k.dw_shift, b, k.T, k.F, k.hid, k.st, k.sf, s);
-                });
+                ExpDwArgs e;
+                e.X = d_x_[cur]; e.D = d_dwo_; e.W = k.pw1.w; e.wstride = k.pw1.stride; e.wscale = k.pw1.scale;
+                e.bexp = k.b1; e.wdw = k.dw_w; e.bdw = k.dw_shift; e.sdw = k.dw_scale; e.n = b;
+                timed("audio_expdw", (double(rows_in) * k.ci + double(rows_out) * k.hid) * 4, s,
+                      [&] { launch_audio_expdw<G>(i, e, s); },
+                      2.0 * k.hid * (double(rows_in) * k.ci + double(rows_out) * 9));
                 check_launch();
                 GemmArgs p2;
                 p2.M = int(rows_out); p2.N = k.co; p2.K = k.hid;

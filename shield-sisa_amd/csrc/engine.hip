@@ -383,7 +383,7 @@ private:
         for (int i = 0; i < 15; ++i) {
             const BlockHost& b = hm.blocks[i];
             xe = std::max(xe, size_t(b.Ho) * b.Wo * b.cfg.cout);
-            if (b.has_expand) ee = std::max(ee, size_t(b.H) * b.W * b.cfg.cexp);
+            if (!kF32 && b.has_expand) ee = std::max(ee, size_t(b.H) * b.W * b.cfg.cexp);
             de = std::max(de, size_t(b.Ho) * b.Wo * b.cfg.cexp);
         }
         xe_ = xe;
@@ -678,20 +678,29 @@ private:
             const Blk& b = blk_[i];
             const long long HWi = (long long)b.H * b.W, HWo = (long long)b.Ho * b.Wo;
             const int act = b.cfg.hs ? ACT_HS : ACT_RELU;
-            const float* dwin = a.X;
-            if (b.has_expand) {
-                GemmArgs p;
-                p.M = int(F * HWi); p.N = b.cfg.cexp; p.K = b.cfg.cin;
-                p.A = a.X; p.lda = b.cfg.cin; p.ldw = b.cfg.cin;
-                p.bias = b.exp_b; p.act = act;
-                p.C = a.E; p.ldc = b.cfg.cexp;
-                gemm("gemm_pw", p, b.exp_w, s);
-                dwin = a.E;
+            if (kF32 && b.has_expand) {   // the expanded map stays in LDS
+                ExpDwArgs e;
+                e.X = a.X; e.D = a.D; e.W = b.exp_w.w; e.bexp = b.exp_b; e.wdw = b.dw_w; e.bdw = b.dw_b; e.n = F;
+                timed("expdw", double(F) * (HWi * b.cfg.cin + HWo * b.cfg.cexp) * TS, s,
+                      [&] { launch_expdw_f32(i + 1, e, s); },
+                      2.0 * F * (double(HWi) * b.cfg.cin + double(HWo) * b.cfg.k * b.cfg.k) * b.cfg.cexp);
+                check_launch();
+            } else {
+                const float* dwin = a.X;
+                if (b.has_expand) {
+                    GemmArgs p;
+                    p.M = int(F * HWi); p.N = b.cfg.cexp; p.K = b.cfg.cin;
+                    p.A = a.X; p.lda = b.cfg.cin; p.ldw = b.cfg.cin;
+                    p.bias = b.exp_b; p.act = act;
+                    p.C = a.E; p.ldc = b.cfg.cexp;
+                    gemm("gemm_pw", p, b.exp_w, s);
+                    dwin = a.E;
+                }
+                timed("dw", double(F) * (HWi + HWo) * b.cfg.cexp * TS, s, [&] {
+                    launch_dw<float>(dwin, a.D, b.dw_w, b.dw_b, F, b.H, b.W, b.cfg.cexp, b.cfg.k, b.cfg.stride, b.Ho, b.Wo, act, s);
+                });
+                check_launch();
             }
-            timed("dw", double(F) * (HWi + HWo) * b.cfg.cexp * TS, s, [&] {
-                launch_dw<float>(dwin, a.D, b.dw_w, b.dw_b, F, b.H, b.W, b.cfg.cexp, b.cfg.k, b.cfg.stride, b.Ho, b.Wo, act, s);
-            });
-            check_launch();
             if (b.cfg.se) {
                 timed("se_pool", double(F) * HWo * b.cfg.cexp * TS, s,
                       [&] { launch_se_pool<float>(a.D, a.se_pool, F, b.Ho, b.Wo, b.cfg.cexp, s); });

@@ -149,6 +149,24 @@ template <typename T> bool launch_ir_strip(int block, const IrArgs& a, int F, hi
 void launch_se_reduce(const float* part, int ntiles, int cexpp, int cexp, int hw, float* pooled, int F,
                       hipStream_t s);
 
+// ---------------------------------------------------------------- expand + depthwise in one kernel (expdw.hip)
+// X [n][H][W][K] -> expand (1x1 weights W [C][K], parts wstride apart, * wscale, + bexp, activation) -> depthwise
+// (wdw [KS * KS][C]) -> D [n][Ho][Wo][C]; H, W, K, C are the block's.
+struct ExpDwArgs {
+    const float* X = nullptr;
+    float* D = nullptr;
+    const void* W = nullptr; long long wstride = 0; float wscale = 1.0f;
+    const float* bexp = nullptr;
+    const float* wdw = nullptr;
+    const float* bdw = nullptr;   // bias (SHIELD-A: BatchNorm shift)
+    const float* sdw = nullptr;   // SHIELD-A: BatchNorm scale
+    int n = 0;                    // frames / windows
+};
+// exact tier, blocks 2..15: bitwise gemm_f32 (bias, activation) + launch_dw
+void launch_expdw_f32(int block, const ExpDwArgs& p, hipStream_t s);
+// SHIELD-A frontend blocks 0..7: the tier's GEMM arithmetic, bias, SiLU; depthwise 3x3 as a sum of products, BatchNorm, SiLU
+template <typename T> void launch_audio_expdw(int block, const ExpDwArgs& p, hipStream_t s);
+
 // ---------------------------------------------------------------- SHIELD-A frontend (engine/audio/frontend.cpp)
 constexpr int kAudioWindowSamples = 160000;              // 10 s of 16 kHz PCM
 constexpr int kAudioMelFrames = 997, kAudioMelBins = 80;  // log-mel image [time][freq]
@@ -168,10 +186,6 @@ void launch_audio_mel(const float* pcm, long long stride, int n, const AudioMelT
 // SiLU
 void launch_audio_stem(const float* mel, const float* w, const float* scale, const float* shift, float* out, int n,
                        hipStream_t s);
-// depthwise 3x3, strides (time st, freq sf) in {1, 2}, padding 1, BatchNorm, SiLU: in [n][T][F][C] ->
-// out [n][(T + st - 1) / st][(F + sf - 1) / sf][C]; w [9][C] (tap 3 kf + kt), C % 4 == 0
-void launch_audio_dw(const float* in, float* out, const float* w, const float* scale, const float* shift, int n,
-                     int T, int F, int C, int st, int sf, hipStream_t s);
 // frequency attention: image [n][125][20][192], attention weights w [192] and bias -> pooled [n][125][192]
 void launch_audio_freq_pool(const float* h, const float* w, float bias, float* pooled, int n, hipStream_t s);
 

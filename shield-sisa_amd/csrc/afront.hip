@@ -1,11 +1,10 @@
 // SHIELD-A frontend kernels for gfx950 (the reference: engine/audio/frontend.cpp): the log-mel frames of a 10 s
-// window, the CNN's stem and the frequency-attention pooling.  Its blocks' expand and depthwise layers are expdw.hip's, the
-// 1x1 projections and the token projection GEMMs of the engine's tiers.  Activations are fp32 in HBM, image layout [time][freq][channel].
+// window and the frequency-attention pooling.  The CNN's stem and its blocks' expand and depthwise layers are expdw.hip's,
+// the 1x1 projections and the token projection GEMMs of the engine's tiers.  Activations are fp32 in HBM, image layout [time][freq][channel].
 //
 // Per element these kernels perform the reference's IEEE operations in its order (the reference is compiled with
 // -ffp-contract=off, and so is this file): the radix-2 FFT's butterflies, the power spectrum, the filterbank fma
-// chain, the stem's fma chain over its nine taps, BatchNorm as a product then a sum, the softmax's running sum.  SiLU
-// (silu_near) and the device's exp and log (softmax, mel energies) are within an ulp or two of glibc's.
+// chain, the softmax's running sum.  The device's exp and log (softmax, mel energies) are within an ulp or two of glibc's.
 #include "dev_common.hpp"
 #include "kernels.hpp"
 
@@ -73,45 +72,6 @@ __global__ void __launch_bounds__(64 * MEL_WAVES) audio_mel_kernel(const float* 
     }
 }
 
-// ---------------------------------------------------------------------------------------------------- stem
-// 3x3 convolution 1 -> 32 channels over the [997][80] log-mel image (zero padding), BatchNorm, SiLU
-// (frontend.cpp:205-212): per output an fma chain from +0 over the taps q = 3 kf + kt (a padding tap adds a zero
-// product, as the reference's zero patch entries do).  Four lanes per pixel, eight channels each.
-__global__ void __launch_bounds__(256) audio_stem_kernel(const float* __restrict__ mel, const float* __restrict__ w,
-                                                         const float* __restrict__ scale,
-                                                         const float* __restrict__ shift, float* __restrict__ out,
-                                                         long long pixels) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= pixels * 4) return;
-    const long long px = i >> 2;
-    const int c0 = int(i & 3) * 8;
-    const long long win = px / (kAudioMelFrames * kAudioMelBins);
-    const int rem = int(px - win * (kAudioMelFrames * kAudioMelBins));
-    const int t = rem / kAudioMelBins, f = rem - t * kAudioMelBins;
-    const float* m = mel + win * (kAudioMelFrames * kAudioMelBins);
-    float patch[9];
-#pragma unroll
-    for (int kf = 0; kf < 3; ++kf)
-#pragma unroll
-        for (int kt = 0; kt < 3; ++kt) {
-            const int ti = t + kt - 1, fi = f + kf - 1;
-            patch[kf * 3 + kt] =
-                (ti >= 0 && ti < kAudioMelFrames && fi >= 0 && fi < kAudioMelBins) ? m[ti * kAudioMelBins + fi] : 0.0f;
-        }
-    float y[8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        float s = 0.0f;
-#pragma unroll
-        for (int q = 0; q < 9; ++q) s = __builtin_fmaf(patch[q], w[(c0 + c) * 9 + q], s);
-        const float v = s * scale[c0 + c] + shift[c0 + c];
-        y[c] = silu_near(v);
-    }
-    float4* o = reinterpret_cast<float4*>(out + px * 32 + c0);
-    o[0] = make_float4(y[0], y[1], y[2], y[3]);
-    o[1] = make_float4(y[4], y[5], y[6], y[7]);
-}
-
 // ---------------------------------------------------------------------------------------------------- attention
 // Frequency attention over the [125][20][192] image (frontend.cpp:222-231), one wave per time step: the 20 logits
 // (an fma chain from +0 over the 192 channels, then + bias), their softmax (running max, exp(l - max), the sum in
@@ -156,14 +116,6 @@ void launch_audio_mel(const float* pcm, long long stride, int n, const AudioMelT
     if (!pcm || !mel || stride < kAudioWindowSamples) throw std::runtime_error("audio mel: bad PCM or window stride");
     hipLaunchKernelGGL(audio_mel_kernel, dim3(cdiv(kAudioMelFrames, MEL_WAVES), (unsigned)n), dim3(64 * MEL_WAVES), 0,
                        s, pcm, stride, tb, mel);
-}
-
-void launch_audio_stem(const float* mel, const float* w, const float* scale, const float* shift, float* out, int n,
-                       hipStream_t s) {
-    if (n <= 0) return;
-    const long long pixels = (long long)n * kAudioMelFrames * kAudioMelBins;
-    hipLaunchKernelGGL(audio_stem_kernel, dim3(cdiv(pixels * 4, 256)), dim3(256), 0, s, mel, w, scale, shift, out,
-                       pixels);
 }
 
 void launch_audio_freq_pool(const float* h, const float* w, float bias, float* pooled, int n, hipStream_t s) {

@@ -149,7 +149,7 @@ private:
             return std::tie(kind, in, ldw, out, n) < std::tie(o.kind, o.in, o.ldw, o.out, o.n);
         }
     };
-    // the frontend runs over chunks of this many windows (its activations: about 28 MB per window)
+    // the frontend runs over chunks of this many windows (its activations: about 14 MB per window)
     static constexpr int kFrontChunk = 16;
     struct FrontBlock {
         int ci, hid, co, sf, st, T, F, To, Fo;
@@ -193,7 +193,7 @@ private:
         stem_scale_ = upl.up(F.stem_scale);
         stem_shift_ = upl.up(F.stem_shift);
         int T = kAudioMelFrames, Fq = kAudioMelBins;
-        size_t xmax = size_t(T) * Fq * 32, dmax = 0;
+        size_t xmax = 0, dmax = 0;
         for (int i = 0; i < 8; ++i) {
             const AudioBlockHost& h = F.blocks[i];
             FrontBlock& b = fblk_[i];
@@ -242,17 +242,15 @@ private:
                   [&] { launch_audio_mel(pcm + w0 * stride, stride, b, mel_tables_, d_mel_, s); });
             check_launch();
             if (w0 == 0 && !dump_dir_.empty()) dump_mel(s);
-            timed("audio_stem", double(b) * kAudioMelFrames * kAudioMelBins * (1 + 32) * 4, s,
-                  [&] { launch_audio_stem(d_mel_, stem_w_, stem_scale_, stem_shift_, d_x_[0], b, s); });
-            check_launch();
             int cur = 0;
             for (int i = 0; i < 8; ++i) {
                 const FrontBlock& k = fblk_[i];
                 const long long rows_in = (long long)b * k.T * k.F, rows_out = (long long)b * k.To * k.Fo;
                 ExpDwArgs e;
-                e.X = d_x_[cur]; e.D = d_dwo_; e.W = k.pw1.w; e.wstride = k.pw1.stride; e.wscale = k.pw1.scale;
+                e.X = i == 0 ? d_mel_ : d_x_[cur]; e.D = d_dwo_; e.W = k.pw1.w; e.wstride = k.pw1.stride; e.wscale = k.pw1.scale;
                 e.bexp = k.b1; e.wdw = k.dw_w; e.bdw = k.dw_shift; e.sdw = k.dw_scale; e.n = b;
-                timed("audio_expdw", (double(rows_in) * k.ci + double(rows_out) * k.hid) * 4, s,
+                if (i == 0) { e.stem_w = stem_w_; e.stem_scale = stem_scale_; e.stem_shift = stem_shift_; }
+                timed("audio_expdw", (double(rows_in) * (i == 0 ? 1 : k.ci) + double(rows_out) * k.hid) * 4, s,
                       [&] { launch_audio_expdw<G>(i, e, s); },
                       2.0 * k.hid * (double(rows_in) * k.ci + double(rows_out) * 9));
                 check_launch();

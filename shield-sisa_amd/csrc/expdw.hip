@@ -17,8 +17,10 @@
 // half types by vector instructions (SiLU, depthwise) and the D stores.  So SiLU is the 16-instruction form, and the next
 // chunk's expand weights are read before the depthwise's stores (a load behind a store waits for it).  Against the
 // expand GEMM and the depthwise kernel apart, which wrote and read E: 32 clips in fp32 11.30 -> 9.36 ms, one clip
-// 1214 -> 1142 us; 128 SHIELD-A windows fp16 13.9 -> 11.5 ms, 5 windows fp32 967 -> 939 us.  16 windows fp16, block 0
-// (997 x 80 x 32 -> 64): 105 us, 0.33 GB of maps; with E 0.65 GB more.
+// 1214 -> 1142 us; 128 SHIELD-A windows fp16 13.9 -> 11.5 ms, 5 windows fp32 967 -> 939 us.  SHIELD-A's first block also
+// computes its input, the stem, from the log-mel tile in LDS, once per band in the fragments' own layout: a stem kernel
+// wrote 163 MB per 16 windows in 113 us (each thread loaded its 72 weights) and the block took 105 us; together 125 us,
+// 128 windows fp16 11.5 -> 10.6 ms, 5 windows fp32 939 -> 907 us.
 #include "dev_common.hpp"
 #include "gemm_f32.hpp"
 #include "kernels.hpp"
@@ -38,7 +40,7 @@ constexpr int ED_WAVES = 8, ED_THREADS = 64 * ED_WAVES;
 constexpr int ED_CS = 16 + 4;   // LDS floats per pixel: the four pixel rows of an accumulator write fall on distinct banks
 
 // Geometry of one block.  MODE: activation and depthwise arithmetic.
-enum { ED_RELU = 0, ED_HS = 1, ED_AUDIO = 2 };
+enum { ED_RELU = 0, ED_HS = 1, ED_AUDIO = 2, ED_STEM = 3 };   // ED_STEM: ED_AUDIO, X computed from the log-mel image
 template <int H_, int W_, int K_, int C_, int KS_, int SY_, int SX_, int MODE_, int BR_, int NI_, int R_, int WGS_ = 1>
 struct EdShape {
     static constexpr int H = H_, W = W_, K = K_, C = C_, KS = KS_, SY = SY_, SX = SX_, MODE = MODE_, BR = BR_, NI = NI_, R = R_,
@@ -50,8 +52,12 @@ struct EdShape {
     static constexpr int CHUNKS = (C + 15) / 16, BANDS = (Ho + BR - 1) / BR;
     static constexpr int GROUPS = (BR + R - 1) / R, UNITS = NI * GROUPS * Wo, WR = (R - 1) * SY + KS;
     // window rows of the last group reach past the tile when R does not divide BR: the LDS tile has them
-    static constexpr int RL = (GROUPS * R - 1) * SY + KS, LDS = NI * RL * WP * ED_CS;
+    static constexpr int RL = (GROUPS * R - 1) * SY + KS, E_LDS = NI * RL * WP * ED_CS;
+    // ED_STEM: after E the band's log-mel rows and columns with a border of one, then the stem's weights [9][32], scale, shift
+    static constexpr bool AUDIO = MODE >= ED_AUDIO, STEM = MODE == ED_STEM;
+    static constexpr int MELW = W + 2, MEL = ((RV + 2) * MELW + 3) / 4 * 4, LDS = E_LDS + (STEM ? MEL + 11 * 32 : 0);
     static_assert(NI == 1 || BR >= Ho, "several images: whole maps");
+    static_assert(!STEM || (K == 32 && NI == 1), "the stem has 32 channels");
 };
 
 // one 16 x 16 x K product in the tier's arithmetic; fragments as the GEMM kernels'
@@ -61,7 +67,7 @@ template <typename T, int K> struct EdMma {   // half types: K steps of 32, spli
     typedef typename Split<T>::V8 V8;
     struct A { V8 v[NS][P]; };
     struct B { V8 v[NS][P]; };
-    static __device__ __forceinline__ void load_a(A& a, const float* row, int g) {
+    template <class X4> static __device__ __forceinline__ void load_a(A& a, X4&& x4, int g) {   // x4(k): X[k .. k + 3]
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
             const int k = 32 * s + 8 * g;
@@ -69,7 +75,7 @@ template <typename T, int K> struct EdMma {   // half types: K steps of 32, spli
 #pragma unroll
             for (int e = 0; e < 8; ++e) x[e] = 0.0f;
             if (K % 32 == 0 || k < K) {
-                const f32x4 lo = ld4(row + k), hi = ld4(row + k + 4);
+                const f32x4 lo = x4(k), hi = x4(k + 4);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     x[e] = lo[e];
@@ -104,10 +110,10 @@ template <int K> struct EdMma<float, K> {   // the reference's K blocks of 64 (g
     static constexpr int NC = (K + 15) / 16;
     struct A { float v[NC][4]; };
     struct B { f32x4 v[NC]; };
-    static __device__ __forceinline__ void load_a(A& a, const float* row, int g) {
+    template <class X4> static __device__ __forceinline__ void load_a(A& a, X4&& x4, int g) {
         f32x4 x[NC];
 #pragma unroll
-        for (int c = 0; c < NC; ++c) x[c] = ld4(row + min(16 * c + 4 * g, K - 4));
+        for (int c = 0; c < NC; ++c) x[c] = x4(min(16 * c + 4 * g, K - 4));
 #pragma unroll
         for (int c = 0; c < NC; ++c) transpose4(x[c], a.v[c]);
     }
@@ -150,15 +156,49 @@ __global__ void __launch_bounds__(ED_THREADS, (std::is_same<T, bf16>::value ? 1 
     const int iy0 = oy0 * S::SY - S::P;                                   // map row of LDS row 0
     const int va = max(iy0, 0), vb = min(S::H, iy0 + S::RI);              // rows inside the map
     const int m_end = imgs * (vb - va) * S::W;                            // pixels (several images: whole maps)
-    const float* x0 = p.X + ((long long)img0 * S::H + va) * (S::W * S::K);
     const int per = (S::CHUNKS + gridDim.y - 1) / gridDim.y;
     const int ch0 = blockIdx.y * per, ch1 = min(S::CHUNKS, ch0 + per);
     if (ch0 >= ch1) return;   // uniform over the workgroup
 
-    typename M::A a[S::MT];
+    typename M::A a[S::MT];   // tiles past the band read its last pixel and are not used
+    if constexpr (S::STEM) {
+        float *mel = E + S::E_LDS, *sw = mel + S::MEL;
+        const float* src = p.X + (long long)img0 * (S::H * S::W);
+        for (int i = tid; i < (vb - va + 2) * S::MELW; i += ED_THREADS) {
+            const int y = va - 1 + i / S::MELW, x = i % S::MELW - 1;
+            mel[i] = y >= 0 && y < S::H && x >= 0 && x < S::W ? src[y * S::W + x] : 0.0f;
+        }
+        for (int i = tid; i < 11 * 32; i += ED_THREADS)
+            sw[i] = i < 288 ? p.stem_w[(i & 31) * 9 + (i >> 5)] : i < 320 ? p.stem_scale[i - 288] : p.stem_shift[i - 320];
+        lds_barrier();
 #pragma unroll
-    for (int t = 0; t < S::MT; ++t)   // tiles past the band read its last pixel and are not used
-        M::load_a(a[t], x0 + (long long)min((wave + ED_WAVES * t) * 16 + r, m_end - 1) * S::K, g);
+        for (int t = 0; t < S::MT; ++t) {
+            const int m = min((wave + ED_WAVES * t) * 16 + r, m_end - 1), row = m / S::W, col = m - row * S::W;
+            float tap[9];   // (kf, kt)
+#pragma unroll
+            for (int q = 0; q < 9; ++q) tap[q] = mel[(row + q % 3) * S::MELW + col + q / 3];
+            M::load_a(a[t], [&](int k) {
+                f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int q = 0; q < 9; ++q) {
+                    const f32x4 w = ld4(sw + q * 32 + k);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) s[e] = __builtin_fmaf(tap[q], w[e], s[e]);
+                }
+                const f32x4 sc = ld4(sw + 288 + k), sh = ld4(sw + 320 + k);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[e] = silu_near(s[e] * sc[e] + sh[e]);
+                return s;
+            }, g);
+        }
+    } else {
+        const float* x0 = p.X + ((long long)img0 * S::H + va) * (S::W * S::K);
+#pragma unroll
+        for (int t = 0; t < S::MT; ++t) {
+            const float* row = x0 + (long long)min((wave + ED_WAVES * t) * 16 + r, m_end - 1) * S::K;
+            M::load_a(a[t], [&](int k) { return ld4(row + k); }, g);
+        }
+    }
     typename M::B b;
     const auto fetch = [&](int ch, float& eb) {   // a chunk's expand weights and bias
         const int n = min(ch * 16 + r, S::C - 1);
@@ -167,7 +207,7 @@ __global__ void __launch_bounds__(ED_THREADS, (std::is_same<T, bf16>::value ? 1 
     };
     float eb_next;
     fetch(ch0, eb_next);
-    for (int i = tid; i < S::LDS / 4; i += ED_THREADS) reinterpret_cast<f32x4*>(E)[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i = tid; i < S::E_LDS / 4; i += ED_THREADS) reinterpret_cast<f32x4*>(E)[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     // LDS position of the lane's first pixel of each tile (of each pixel where a row is no multiple of four)
     constexpr int PI = S::W % 4 == 0 ? 1 : 4;
     int eo[S::MT][PI];
@@ -204,7 +244,7 @@ __global__ void __launch_bounds__(ED_THREADS, (std::is_same<T, bf16>::value ? 1 
         float w[S::KS * S::KS];
 #pragma unroll
         for (int q = 0; q < S::KS * S::KS; ++q) w[q] = p.wdw[q * S::C + cc];
-        const float db = p.bdw[cc], ds = S::MODE == ED_AUDIO ? p.sdw[cc] : 1.0f;
+        const float db = p.bdw[cc], ds = S::AUDIO ? p.sdw[cc] : 1.0f;
 #pragma unroll
         for (int t = 0; t < S::MT; ++t) {
             if ((wave + ED_WAVES * t) * 16 >= m_end) break;   // uniform over the wave
@@ -244,7 +284,7 @@ __global__ void __launch_bounds__(ED_THREADS, (std::is_same<T, bf16>::value ? 1 
 #pragma unroll
             for (int o = 0; o < S::R; ++o) {
                 float s = 0.0f, v;
-                if constexpr (S::MODE == ED_AUDIO) {   // columns (frequency) outer, rows (time) inner; product, then sum
+                if constexpr (S::AUDIO) {   // columns (frequency) outer, rows (time) inner; product, then sum
 #pragma unroll
                     for (int x = 0; x < S::KS; ++x)
 #pragma unroll
@@ -303,7 +343,7 @@ typedef EdShape<12, 20, 80, 480, 3, 1, 1, ED_HS, 12, 1, 4> B11;
 typedef EdShape<12, 20, 112, 672, 3, 1, 1, ED_HS, 12, 1, 2, 2> B12;
 typedef EdShape<12, 20, 112, 672, 5, 2, 2, ED_HS, 6, 1, 2> B13;
 typedef EdShape<6, 10, 160, 960, 5, 1, 1, ED_HS, 6, 2, 2> B14;
-typedef EdShape<997, 80, 32, 64, 3, 2, 2, ED_AUDIO, 4, 1, 2, 2> A0;
+typedef EdShape<997, 80, 32, 64, 3, 2, 2, ED_STEM, 4, 1, 2, 2> A0;
 typedef EdShape<499, 40, 48, 96, 3, 1, 1, ED_AUDIO, 10, 1, 5, 2> A1;   // fp32
 typedef EdShape<499, 40, 48, 96, 3, 1, 1, ED_AUDIO, 7, 1, 2, 2> A1H;   // half types
 typedef EdShape<499, 40, 48, 96, 3, 2, 2, ED_AUDIO, 5, 1, 5, 2> A2;
@@ -338,6 +378,7 @@ void launch_expdw_f32(int block, const ExpDwArgs& p, hipStream_t s) {
 }
 template <typename T> void launch_audio_expdw(int block, const ExpDwArgs& p, hipStream_t s) {
     check(p);
+    if (block == 0 && (!p.stem_w || !p.stem_scale || !p.stem_shift)) throw std::runtime_error("expdw: bad operands");
     switch (block) {
     case 0: launch_shape<T, A0>(p, s); return;
     case 1: launch_shape<T, std::conditional_t<std::is_same<T, float>::value, A1, A1H>>(p, s); return;

@@ -160,11 +160,14 @@ struct ExpDwArgs {
     const float* wdw = nullptr;
     const float* bdw = nullptr;   // bias (SHIELD-A: BatchNorm shift)
     const float* sdw = nullptr;   // SHIELD-A: BatchNorm scale
+    const float *stem_w = nullptr, *stem_scale = nullptr, *stem_shift = nullptr;   // SHIELD-A block 0: see below
     int n = 0;                    // frames / windows
 };
 // exact tier, blocks 2..15: bitwise gemm_f32 (bias, activation) + launch_dw
 void launch_expdw_f32(int block, const ExpDwArgs& p, hipStream_t s);
 // SHIELD-A frontend blocks 0..7: the tier's GEMM arithmetic, bias, SiLU; depthwise 3x3 as a sum of products, BatchNorm, SiLU
+// Block 0 computes its input itself: X is the log-mel image [n][997][80], on it the 3x3 stem (w [32][9], tap 3 kf + kt, an
+// fma chain over the taps), BatchNorm scale / shift, SiLU.
 template <typename T> void launch_audio_expdw(int block, const ExpDwArgs& p, hipStream_t s);
 
 // ---------------------------------------------------------------- SHIELD-A frontend (engine/audio/frontend.cpp)
@@ -182,10 +185,6 @@ struct AudioMelTables {
 };
 // PCM windows (window w at pcm + w * stride, stride >= 160,000 samples) -> normalised log-mel [n][997][80]
 void launch_audio_mel(const float* pcm, long long stride, int n, const AudioMelTables& tb, float* mel, hipStream_t s);
-// log-mel [n][997][80] -> stem image [n][997][80][32]: 3x3 conv (w [32][9], tap 3 kf + kt), BatchNorm scale/shift,
-// SiLU
-void launch_audio_stem(const float* mel, const float* w, const float* scale, const float* shift, float* out, int n,
-                       hipStream_t s);
 // frequency attention: image [n][125][20][192], attention weights w [192] and bias -> pooled [n][125][192]
 void launch_audio_freq_pool(const float* h, const float* w, float bias, float* pooled, int n, hipStream_t s);
 

@@ -157,7 +157,7 @@ int shv_hip_set_dump_dir(shv_hip_model* m, const char* dir);
  * create repacks W on the device (synchronising `stream`); NULL + last_error on failure (fp16 / bf16 need k % 8 == 0).
  * run: variant 0 = the engine's own kernel choice; fp32: 1 GEMV, 2 tiled, 3 K blocks in parallel (1-3: the CPU
  * engine's operation order; 3 allocates its workspace of ceil(k / 64) * m * n floats and synchronises `stream`),
- * 4 the fp32 matrix cores (k % 4 == 0), 5 narrow (CPU order; the (k, n) shapes of blocks 1-6 only: 16x16, 16x64,
+ * 4 the fp32 matrix cores (CPU order, k % 4 == 0), 5 narrow (CPU order; the (k, n) shapes of blocks 1-6 only: 16x16, 16x64,
  * 64x24, 24x72, 72x24, 72x40, 40x120, 120x40), 6 column chunks (CPU order, k <= 1024, k % 4 == 0); fp16 / bf16:
  * 1 small-M, 2..6 direct with
  * 1..5 column tiles per wave, 7 LDS-staged, 8 streaming (n <= 160).  Returns 0, or -1 + last_error.  Asynchronous on

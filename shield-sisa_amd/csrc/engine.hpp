@@ -23,11 +23,11 @@
 namespace shv {
 
 // The exact tier's arithmetic in the sequence stages.  The CNN always performs the reference CPU engine's operation
-// order (its tokens are bitwise the reference's).  By default the all-row sequence GEMMs run on the fp32 matrix cores
-// and the delta rule splits each value column's keys over lane groups (fp32 values and operations, in an order of
-// this engine's own); SHV_HIP_F32_CPU_ORDER=1 at load keeps the reference's order there too (VALU GEMMs in K blocks
-// of 64, the 64-key fma chains), so that every stage output is the reference's: the check that pins the sequence
-// stage code to the reference.
+// order (its tokens are bitwise the reference's), and so do the sequence GEMMs (K blocks of 64, on the fp32 matrix
+// cores).  By default the delta rule is the chunked scan (fp32 values and operations, in an order of this engine's
+// own); SHV_HIP_F32_CPU_ORDER=1 at load keeps the reference's order there too (token by token, the 64-key fma
+// chains), so that every stage output is the reference's: the check that pins the sequence stage code to the
+// reference.
 inline bool f32_cpu_order_requested() {
     const char* e = std::getenv("SHV_HIP_F32_CPU_ORDER");
     return e && *e && std::strcmp(e, "0") != 0;
@@ -181,8 +181,7 @@ public:
     PwGemm(const PwGemm&) = delete;
     PwGemm& operator=(const PwGemm&) = delete;
     // variant: kernel choice (0 = the engine's own: for fp32 the CNN's, the reference CPU order); see
-    // gemm_f32_variant / gemm_mfma_variant; fp32 4 = the fp32 matrix cores (gemm_f32_mfma, the sequence stages'
-    // kernel)
+    // gemm_f32_variant / gemm_mfma_variant; fp32 4 = the fp32 matrix cores whatever M (gemm_f32_mfma)
     void run(const float* A, long long M, const float* bias, int act, float* C, int variant, hipStream_t s) const;
     Precision precision() const { return prec_; }
 

@@ -1342,15 +1342,18 @@ __global__ void __launch_bounds__(64 * MFMA_WAVES, 2) gemm_stream_kernel(GemmArg
                       [&](int i, int j) { return acc[mt][j][i]; });
 }
 
-// Wide GEMM: large M, short K (<= 256), many columns (the config-2 expand M x 160 -> 960, the audio frontend's
-// 1x1 layers).  A workgroup (4 waves) takes 64 rows: their K values are loaded once (16-byte loads), split into the
-// operand parts and staged in LDS, where every wave reads them; wave w then walks the 16-column tiles w, w + 4, ...
-// of N, each a 64 x 16 output block of 4 accumulators.  A tile's weight fragments for all KS K steps are loaded in
-// one go one tile ahead (two register sets alternating with the tile parity), so a wave waits on L2 once per tile,
-// not once per K step.  Results go through the wave's LDS region and leave as whole 64-byte row pieces,
+// Wide GEMM: large M, short K (<= 256), many columns (the config-2 expand M x 160 -> 960, the layer path's wide
+// expands).  A workgroup (4 waves) takes 64 rows: their K values are loaded once (16-byte loads), split into the
+// operand parts and staged in LDS, where every wave reads them; the 16-column tiles of N go in groups of GR over the
+// waves, two tiles at a time, each a 64 x 16 output block of 4 accumulators.  The two tiles' weight fragments for all KS
+// K steps stay in registers, a step's loaded for the next two as soon as its products are done, so that a wave never
+// waits on L2.  Results go through the wave's LDS region and leave as whole 64-byte row pieces,
 // non-temporal.  A is read from HBM exactly once (the direct and LDS-tiled kernels re-read it once per column block:
 // 7-12 times at N = 960).  Per output: K steps of 32 in increasing order, the split products in mfma_split's order,
 // the accumulator from +0, epi_value's epilogue -- bitwise the other MFMA kernels' results.
+// Bound by the CU's LDS (A fragments, C staging) and vector instructions ahead of HBM.  Two tiles per A fragment instead
+// of one halve its LDS reads (40 KB per 64 x 16 outputs at K 160): M 125,440, N 960, K 160 in fp16 196 -> 185 us
+// (2.9 -> 3.0 TB/s; its HBM time about 110 us).
 constexpr int WD_ROWS = 64, WD_KMAX = 256, WD_PAD = 8, WD_SLD = 64 + 4;
 template <typename T, int KS, int GR>
 __global__ void __launch_bounds__(256, 2) gemm_wide_kernel(GemmArgs p) {
@@ -1380,36 +1383,44 @@ __global__ void __launch_bounds__(256, 2) gemm_wide_kernel(GemmArgs p) {
     lds_barrier();
     const T* W = static_cast<const T*>(p.W);
     const int tiles = (p.N + 15) / 16;
-    // tile t's fragments for every K step: lane chunk k = 32 ks + 8 g (zero past K, read at a valid address)
-    const auto load_tile = [&](V8 (&dst)[KS][P], int t) {
+    // tile t's fragments of K step ks: lane chunk k = 32 ks + 8 g (past K, in the last step only: read at a valid address,
+    // zeroed where it is used)
+    const bool last_in = (KS - 1) * 32 + g * 8 < p.K;
+    const auto load_step = [&](V8 (&dst)[P], int t, int ks) {
         const T* wrow = W + (long long)min(t * 16 + r, p.N - 1) * p.ldw + g * 8;
+        const int k = ks < KS - 1 || last_in ? ks * 32 : 0;
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const bool kin = ks * 32 + g * 8 < p.K;
-#pragma unroll
-            for (int q = 0; q < P; ++q) {
-                const V8 v = load_part8<T>(wrow + q * p.wstride + (kin ? ks * 32 : 0));
-                dst[ks][q] = kin ? v : V8{};
-            }
-        }
+        for (int q = 0; q < P; ++q) dst[q] = load_part8<T>(wrow + q * p.wstride + k);
     };
     float* wt = Cs + wave * 16 * WD_SLD;
-    // one 16-column tile's 64 x 16 outputs into acc (4 row tiles), from its prefetched weight fragments
-    const auto tile = [&](f32x4 (&acc)[4], const V8 (&wf)[KS][P]) {
+    // two 16-column tiles' 64 x 16 outputs into acc0 / acc1 (4 row tiles each): every A fragment read from LDS serves
+    // both.  A K step's weight registers are loaded for the next pair (tiles n0, n1) as soon as its products are done,
+    // a whole pair ahead of their use.
+    const auto pair = [&](f32x4 (&acc0)[4], f32x4 (&acc1)[4], V8 (&w0)[KS][P], V8 (&w1)[KS][P], bool more, int n0, int n1) {
 #pragma unroll
-        for (int mt = 0; mt < 4; ++mt) acc[mt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int mt = 0; mt < 4; ++mt) acc0[mt] = acc1[mt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
+            if (ks == KS - 1 && !last_in) {
+#pragma unroll
+                for (int q = 0; q < P; ++q) w0[ks][q] = w1[ks][q] = V8{};
+            }
 #pragma unroll
             for (int mt = 0; mt < 4; ++mt) {
                 V8 a[P];
 #pragma unroll
                 for (int q = 0; q < P; ++q)
                     a[q] = *reinterpret_cast<const V8*>(As + (q * WD_ROWS + mt * 16 + r) * ld + ks * 32 + g * 8);
-                acc[mt] = mfma_split<T>(a, wf[ks], acc[mt]);
+                acc0[mt] = mfma_split<T>(a, w0[ks], acc0[mt]);
+                acc1[mt] = mfma_split<T>(a, w1[ks], acc1[mt]);
             }
             // keeps the compiler from hoisting every K step's A fragment reads ahead of the products
-            asm volatile("" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3])::"memory");
+            asm volatile("" : "+v"(acc0[0]), "+v"(acc0[1]), "+v"(acc0[2]), "+v"(acc0[3]), "+v"(acc1[0]), "+v"(acc1[1]),
+                         "+v"(acc1[2]), "+v"(acc1[3])::"memory");
+            if (more) {
+                load_step(w0[ks], n0, ks);
+                load_step(w1[ks], n1, ks);
+            }
         }
     };
     // a group's 64 x 16 GR outputs (tiles j < GR of columns nbase + 16 j ..): per 16-row block through the wave's
@@ -1482,27 +1493,26 @@ __global__ void __launch_bounds__(256, 2) gemm_wide_kernel(GemmArgs p) {
         default: go_act(std::integral_constant<int, ACT_NONE>{}); break;
         }
     };
-    // wave w takes the GR-tile groups w, w + 4, ...; its tiles' weights alternate between two register sets, the
-    // next tile's loads in flight while one computes
+    // wave w takes the GR-tile groups w, w + 4, ..., a pair of tiles at a time
     static_assert(GR == 2 || GR == 4, "groups of 2 or 4 tiles");
     const int groups = (tiles + GR - 1) / GR;
     V8 w0[KS][P], w1[KS][P];
     const auto tile_of = [&](int gi, int j) { return min(gi * GR + j, tiles - 1); };   // past N: recomputes the last
-    if (wave < groups) load_tile(w0, tile_of(wave, 0));
+    if (wave < groups) {
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            load_step(w0[ks], tile_of(wave, 0), ks);
+            load_step(w1[ks], tile_of(wave, 1), ks);
+        }
+    }
     for (int gi = wave; gi < groups; gi += 4) {
         f32x4 acc[GR][4];
-        load_tile(w1, tile_of(gi, 1));
-        tile(acc[0], w0);
+        const int gn = gi + 4;
         if constexpr (GR == 4) {
-            load_tile(w0, tile_of(gi, 2));
-            tile(acc[1], w1);
-            load_tile(w1, tile_of(gi, 3));
-            tile(acc[2], w0);
-            if (gi + 4 < groups) load_tile(w0, tile_of(gi + 4, 0));
-            tile(acc[3], w1);
+            pair(acc[0], acc[1], w0, w1, true, tile_of(gi, 2), tile_of(gi, 3));
+            pair(acc[2], acc[3], w0, w1, gn < groups, tile_of(gn, 0), tile_of(gn, 1));
         } else {
-            if (gi + 4 < groups) load_tile(w0, tile_of(gi + 4, 0));
-            tile(acc[1], w1);
+            pair(acc[0], acc[1], w0, w1, gn < groups, tile_of(gn, 0), tile_of(gn, 1));
         }
         store_group(acc, gi * GR * 16);
     }

@@ -15,6 +15,7 @@
 //   K advances in steps of 32 in increasing order; a K tail is zero-filled, never split across waves.
 #include "dev_common.hpp"
 #include "gemm_epi.hpp"
+#include "gemm_reach.hpp"
 #include "kernels.hpp"
 #include "mfma.hpp"
 
@@ -1383,12 +1384,12 @@ __global__ void __launch_bounds__(256, 2) gemm_wide_kernel(GemmArgs p) {
     lds_barrier();
     const T* W = static_cast<const T*>(p.W);
     const int tiles = (p.N + 15) / 16;
-    // tile t's fragments of K step ks: lane chunk k = 32 ks + 8 g (past K, in the last step only: read at a valid address,
+    // tile t's fragments of K step ks: lane chunk k = 32 ks + 8 g (past K, in the last step only: another of the row's,
     // zeroed where it is used)
     const bool last_in = (KS - 1) * 32 + g * 8 < p.K;
     const auto load_step = [&](V8 (&dst)[P], int t, int ks) {
         const T* wrow = W + (long long)min(t * 16 + r, p.N - 1) * p.ldw + g * 8;
-        const int k = ks < KS - 1 || last_in ? ks * 32 : 0;
+        const int k = wide_step(KS, ks, g, ks < KS - 1 || last_in);
 #pragma unroll
         for (int q = 0; q < P; ++q) dst[q] = load_part8<T>(wrow + q * p.wstride + k);
     };

@@ -379,8 +379,21 @@ Plan plan(const GemmArgs& p, int swiglu) {
     // the waves; measured in us, tile / split 2 x 2 / split 1 x 1: 1284 x 2316 x 384 (525 tiles) 41 / 46 / 69, 630 x 2316
     // x 384 (250) 29 / 26 / 37, 1200 x 960 x 160 (190) 10.4 / 13.1 / 16.6, 1200 x 160 x 960 (38) 30 / 12.2 / 14.8,
     // 321 x 384 x 768 (24 tiles, 132 2 x 2s) 29 / 10.8 / 9.7.
+    // One block of rows is split however many columns there are, since the split kernel's tiles hold fewer padding rows and
+    // have their K blocks in flight at once: tile / split 2 x 2 at 5 x 30000 x 64 31.9 / 5.9, 32 x 30000 x 960 262 / 37, 64 x
+    // 100000 x 256 257 / 58.
     const long long wgs = (long long)cdiv(p.M, 64) * nb;
-    if (wgs >= 256 || (nkb <= 3 && wgs >= 128) || nkb > 16) return {false, 4, wn};
+    const bool one = p.M <= 64;
+    if (!one && (wgs >= 256 || (nkb <= 3 && wgs >= 128))) return {false, 4, wn};
+    // Past 16 K blocks only the smallest tile's block sums fit the LDS.  Its operands are read once per 16 rows and columns,
+    // so it is the faster one for few tiles only; tile / split 1 x 1: 5 x 384 x 1100 (24 16 x 16s) 39 / 7.2, 20 x 960 x 2048
+    // (120) 68 / 11, 64 x 30000 x 2048 (one block of rows) 549 / 215, 1000 x 384 x 2052 (1512) 70 / 43, 600 x 960 x 2048
+    // (2280) 70 / 67, 600 x 960 x 4096 133 / 149, 2000 x 384 x 1100 (3000) 40 / 48.
+    if (nkb > 16) {
+        const int nt = swiglu == 2 ? 2 : 1;
+        if (nkb * nt > 64 || (!one && (long long)cdiv(p.M, 16) * tiles > 1536)) return {false, 4, wn};
+        return {true, 1, nt};
+    }
     if ((long long)cdiv(p.M, 32) * cdiv(tiles, 2) >= 160) return {true, 2, 2};
     return {true, 1, swiglu == 2 ? 2 : 1};
 }

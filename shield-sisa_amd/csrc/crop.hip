@@ -91,23 +91,11 @@ template <int N> __device__ __forceinline__ void load_bytes(GBytes p, unsigned (
     for (int d = 0; d < load_words(N); ++d) w[d] = *reinterpret_cast<const AS_GLOBAL UWord*>(p + 4 * d);
 }
 
-// BT.601 limited-range coefficients of ffmpeg's yuv2rgb tables (contrast = saturation = 1 << 16, brightness 0),
-// rounded to 16 bits as av_clip_int16((x + 2^15) >> 16): Y 76309 (= 65536 * 255 / 219) and the inverse-table
-// entries 104597 (V->R), 132201 (U->B), -25675 (U->G), -53279 (V->G), each times 2^13; Y offset 16 << 19
-struct Yuv {
-    int y_coeff, vr, ub, ug, vg, y_off, uv_off;
-};
-__device__ __forceinline__ int sat16(int v) { return v < -32768 ? -32768 : (v > 32767 ? 32767 : v); }
-__device__ __forceinline__ int mulhi16(int a, int b) { return (a * b) >> 16; }
-__device__ __forceinline__ int sat8(int v) { return v < 0 ? 0 : (v > 255 ? 255 : v); }
-__device__ __forceinline__ void yuv_px(const Yuv& k, int y, int u, int v, float (&o)[3]) {
-    const int yp = int(short((y << 3) - k.y_off));
-    const int up = sat16((u << 3) - k.uv_off), vp = sat16((v << 3) - k.uv_off);
-    const int yy = mulhi16(yp, k.y_coeff);
-    const int cg = sat16(mulhi16(up, k.ug) + mulhi16(vp, k.vg));
-    o[0] = float(sat8(sat16(yy + mulhi16(vp, k.vr))));
-    o[1] = float(sat8(sat16(yy + cg)));
-    o[2] = float(sat8(sat16(yy + mulhi16(up, k.ub))));
+__device__ __forceinline__ void yuv_px(int y, int u, int v, float (&o)[3]) {
+    const int yy = yuv_luma(y);
+    o[0] = float(yuv_sat8(yy + yuv_red(v)));
+    o[1] = float(yuv_sat8(yy + yuv_green(u, v)));
+    o[2] = float(yuv_sat8(yy + yuv_blue(u)));
 }
 
 // Native sources.  Row: where a source row starts (uniform).  Raw<K>: what a thread loads of a row for K pixels from
@@ -135,7 +123,6 @@ struct I420Src {   // converted per pixel
     GBytes Y, U, V;
     long long ys, us, vs;
     int h;
-    Yuv k;
     struct Row { GBytes y, u, v; };
     template <int K> struct Raw { unsigned y[load_words(K)], u[load_words(chroma_samples(K))], v[load_words(chroma_samples(K))]; };
     __device__ bool last(int y) const { return (y >> 1) == ((h + 1) >> 1) - 1; }
@@ -144,25 +131,28 @@ struct I420Src {   // converted per pixel
     }
     template <int K> __device__ void load(int x, const Row& q, Raw<K>& r) const {
         constexpr int C = chroma_samples(K);
-        static_assert(load_words(C) == 1, "tap() picks the chroma samples out of one word");
         load_bytes<K>(q.y + unsigned(x), r.y);
         load_bytes<C>(q.u + (unsigned(x) >> 1), r.u);
         load_bytes<C>(q.v + (unsigned(x) >> 1), r.v);
     }
     template <int K> __device__ void tap(const Raw<K>& r, int x, int i, float (&o)[3]) const {
-        const int sh = 8 * ((i + (x & 1)) >> 1);
-        yuv_px(k, int(byte_of(r.y, i)), int((r.u[0] >> sh) & 255u), int((r.v[0] >> sh) & 255u), o);
+        const int odd = x & 1;
+        const auto chroma = [&](const unsigned* c) {
+            if constexpr (load_words(chroma_samples(K)) == 1) return (c[0] >> (8 * ((i + odd) >> 1))) & 255u;
+            return odd ? byte_of(c, (i + 1) >> 1) : byte_of(c, i >> 1);
+        };
+        yuv_px(int(byte_of(r.y, i)), int(chroma(r.u)), int(chroma(r.v)), o);
     }
     __device__ void pixel(int x, const Row& q, float (&o)[3]) const {
-        yuv_px(k, q.y[unsigned(x)], q.u[unsigned(x) >> 1], q.v[unsigned(x) >> 1], o);
+        yuv_px(q.y[unsigned(x)], q.u[unsigned(x) >> 1], q.v[unsigned(x) >> 1], o);
     }
 };
 struct RingSrc {   // canvas rows in the LDS ring, one word (R, G, B) per pixel
     const unsigned* px;
-    int pw;
+    int width;   // of a row
     struct Row { const unsigned* p; };
     template <int K> struct Raw { unsigned px[K]; };
-    __device__ Row row(int y) const { return {px + (y % CROP_RING) * pw}; }
+    __device__ Row row(int y) const { return {px + (y % CROP_RING) * width}; }
     template <int K> __device__ void load(int x, const Row& q, Raw<K>& r) const {
 #pragma unroll
         for (int k = 0; k < K; ++k) r.px[k] = q.p[x + k];
@@ -212,6 +202,18 @@ template <int K, class Src> struct Rows {
         }
     }
 };
+// the row pass of K pixels
+template <int K, class Src>
+__device__ __forceinline__ void row_pass(const Src& src, const typename Src::template Raw<K>& raw, int x0, const float* w,
+                                         float (&t)[3]) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        float v[3];
+        src.template tap<K>(raw, x0, k, v);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) t[c] = k == 0 ? v[c] * w[k] : t[c] + v[c] * w[k];
+    }
+}
 // one output pixel of those rows: first source column x0, column weights w
 template <int K, int FIN, class Src>
 __device__ __forceinline__ unsigned resize_px(const Rows<K, Src>& rows, const Src& src, int x0, const float* w, float fscale) {
@@ -222,76 +224,109 @@ __device__ __forceinline__ unsigned resize_px(const Rows<K, Src>& rows, const Sr
 #pragma unroll
     for (int j = 0; j < K; ++j) {
         float t[3];
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-            float v[3];
-            src.template tap<K>(raw[j], x0, k, v);
-#pragma unroll
-            for (int c = 0; c < 3; ++c) t[c] = k == 0 ? v[c] * w[k] : t[c] + v[c] * w[k];
-        }
+        row_pass<K>(src, raw[j], x0, w, t);
         col.add(j == 0, rows.b[j], t);
     }
     return col.finish(fscale);
 }
-// output pixel (x, y) of any plan, source pixel by source pixel, all inside the source
-template <int FIN, class Src>
-__device__ __forceinline__ unsigned resize_any_fin(const PlanDev& p, const Src& src, int x, int y) {
-    const auto xw = (const AS_GLOBAL float*)p.xw;
-    const int x0 = ((const AS_GLOBAL int*)p.xoff)[x];
+// the same for wide K, two rows at a time (all of them at once took up to 243 registers)
+template <int K, int FIN, class Src>
+__device__ __forceinline__ unsigned resize_px_wide(const PlanDev& p, const Src& src, int y, int x0, const float* w) {
     Column<FIN> col;
-    for (int j = 0; j < p.K; ++j) {
-        const typename Src::Row row = src.row(((const AS_CONST int*)p.ysi)[y * p.K + j]);
-        float t[3] = {0.0f, 0.0f, 0.0f};
-        for (int k = 0; k < p.K; ++k) {
-            float v[3];
-            src.pixel(min(x0 + k, p.sw - 1), row, v);
-            const float a = xw[x * p.K + k];
-#pragma unroll
-            for (int c = 0; c < 3; ++c) t[c] = t[c] + v[c] * a;
-        }
-        col.add(j == 0, ((const AS_CONST float*)p.yw)[y * p.K + j], t);
+#pragma unroll 2
+    for (int j = 0; j < K; ++j) {
+        typename Src::template Raw<K> raw;
+        src.template load<K>(x0, src.row(((const AS_CONST int*)p.ysi)[y * K + j]), raw);
+        float t[3];
+        row_pass<K>(src, raw, x0, w, t);
+        col.add(j == 0, ((const AS_CONST float*)p.yw)[y * K + j], t);
     }
     return col.finish(p.fscale);
 }
-template <class Src> __device__ __forceinline__ unsigned resize_any(const PlanDev& p, const Src& src, int x, int y) {
+// output pixel (x, y) of any plan, source pixel by source pixel, all inside the source; x and y may differ by thread
+template <int UNROLL, int FIN, class Src>
+__device__ __forceinline__ unsigned resize_any_fin(const PlanDev& p, const Src& src, int x, int y) {
+    const auto xw = (const AS_GLOBAL float*)p.xw + x * p.K;
+    const auto ysi = (const AS_GLOBAL int*)p.ysi + y * p.K;
+    const auto yw = (const AS_GLOBAL float*)p.yw + y * p.K;
+    const int x0 = ((const AS_GLOBAL int*)p.xoff)[x];
+    Column<FIN> col;
+    for (int j = 0; j < p.K; ++j) {
+        const typename Src::Row row = src.row(ysi[j]);
+        float t[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll UNROLL
+        for (int k = 0; k < p.K; ++k) {
+            float v[3];
+            src.pixel(min(x0 + k, p.sw - 1), row, v);
+            const float a = xw[k];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) t[c] = t[c] + v[c] * a;
+        }
+        col.add(j == 0, yw[j], t);
+    }
+    return col.finish(p.fscale);
+}
+template <int UNROLL, class Src> __device__ __forceinline__ unsigned resize_any(const PlanDev& p, const Src& src, int x, int y) {
     switch (p.fin) {
-    case FIN_QUARTER: return resize_any_fin<FIN_QUARTER>(p, src, x, y);
-    case FIN_LINEAR: return resize_any_fin<FIN_LINEAR>(p, src, x, y);
-    default: return resize_any_fin<FIN_SCALE>(p, src, x, y);
+    case FIN_QUARTER: return resize_any_fin<UNROLL, FIN_QUARTER>(p, src, x, y);
+    case FIN_LINEAR: return resize_any_fin<UNROLL, FIN_LINEAR>(p, src, x, y);
+    default: return resize_any_fin<UNROLL, FIN_SCALE>(p, src, x, y);
     }
 }
 
 constexpr int CROP_THREADS = CROP_W, CROP_PASS = 1280 / CROP_THREADS;   // canvas columns per thread
 
-// Canvas rows ya .. yb - 1 of the patch into the ring.  A thread keeps its (up to four) columns' taps for the whole band.
+// The patch columns of a workgroup: pa .. pb in the ring, of which la .. lb lie on the frame and the others under its
+// letterbox bars (zero in every ring row, written once).
+struct Span {
+    int pa, pb, la, lb;
+    __device__ int width() const { return pb - pa; }
+    __device__ int live() const { return lb - la; }
+};
+// A thread's (up to four) live columns' taps, kept for the whole band.
 template <int K> struct Columns {
     int x0[CROP_PASS];
     float w[CROP_PASS][K ? K : 1];
 };
+// Canvas rows ya .. yb - 1 of the patch into the ring.
 template <int K, int FIN, class Src>
-__device__ __forceinline__ void fill_rows(const JobDev& j, const PlanDev& p, const Src& src, const Columns<K>& cs, int ya,
-                                          int yb, unsigned* ring) {
-    const int passes = (j.pw + CROP_THREADS - 1) / CROP_THREADS, xa = j.px0 - j.left;
-    const bool inside = xa >= 0 && xa + j.pw <= j.new_w;   // no letterbox bar left or right of the patch
+__device__ __forceinline__ void fill_rows(const JobDev& j, const PlanDev& p, const Src& src, const Columns<K>& cs,
+                                          const Span& sp, int ya, int yb, unsigned* ring) {
+    const int live = sp.live(), xa = j.px0 + sp.la - j.left;   // column of the resized frame of the first live one
+    if (live <= 0) return;
+    unsigned* base = ring + (sp.la - sp.pa);
+    if constexpr (K == 0) {   // rows and columns together: few of them may be live
+        for (int i = threadIdx.x; i < (yb - ya) * live; i += CROP_THREADS) {
+            const int r = ya + i / live, px = i % live, y = r + j.py0 - j.top;
+            base[(r % CROP_RING) * sp.width() + px] = y >= 0 && y < j.new_h ? resize_any<4>(p, src, xa + px, y) : 0u;
+        }
+        return;
+    }
     for (int r = ya; r < yb; ++r) {
         const int y = r + j.py0 - j.top;   // row of the resized frame; outside it the letterbox bars
-        unsigned* row = ring + (r % CROP_RING) * j.pw;
+        unsigned* row = base + (r % CROP_RING) * sp.width();
         const bool bar = y < 0 || y >= j.new_h;
-        if (K > 0 && !bar && !src.last(((const AS_CONST int*)p.ysi)[y * p.K + p.K - 1])) {
+        if (!bar && !src.last(((const AS_CONST int*)p.ysi)[y * p.K + p.K - 1])) {
             if constexpr (K > 0) {
-                const Rows<K, Src> rows(p, src, y);
+                // uniform passes; a column past the last live one is computed (from its clamp) and dropped
+                const auto passes = [&](auto pixel) {
 #pragma unroll
-                for (int q = 0; q < CROP_PASS; ++q) {
-                    if (q >= passes) break;   // uniform; a column past the patch is computed (from its clamp) and dropped
-                    const int px = threadIdx.x + CROP_THREADS * q;
-                    unsigned v = resize_px<K, FIN>(rows, src, cs.x0[q], cs.w[q], p.fscale);
-                    if (!inside) v = xa + px >= 0 && xa + px < j.new_w ? v : 0u;
-                    if (px < j.pw) row[px] = v;
+                    for (int q = 0; q < CROP_PASS; ++q) {
+                        if (CROP_THREADS * q >= live) break;
+                        const int px = threadIdx.x + CROP_THREADS * q;
+                        const unsigned v = pixel(cs.x0[q], cs.w[q]);
+                        if (px < live) row[px] = v;
+                    }
+                };
+                if constexpr (K <= CROP_KMAX) {
+                    const Rows<K, Src> rows(p, src, y);
+                    passes([&](int x0, const float* w) { return resize_px<K, FIN>(rows, src, x0, w, p.fscale); });
+                } else {
+                    passes([&](int x0, const float* w) { return resize_px_wide<K, FIN>(p, src, y, x0, w); });
                 }
             }
         } else {
-            for (int px = threadIdx.x; px < j.pw; px += CROP_THREADS)
-                row[px] = !bar && xa + px >= 0 && xa + px < j.new_w ? resize_any(p, src, xa + px, y) : 0u;
+            for (int px = threadIdx.x; px < live; px += CROP_THREADS) row[px] = bar ? 0u : resize_any<1>(p, src, xa + px, y);
         }
     }
 }
@@ -319,36 +354,50 @@ __device__ __forceinline__ unsigned out_px_any(const PlanDev& p, const RingSrc& 
 
 template <int K, int FIN, class Src>
 __device__ __forceinline__ void crop_band(const JobDev& j, const PlanDev& np, const PlanDev& cp, const Src& src, int oy0,
-                                          int oy1, unsigned* ring, uint8_t* out) {
+                                          int oy1, int oc0, int cols, unsigned* ring, uint8_t* out) {
+    const auto cxoff = (const AS_CONST int*)cp.xoff;
+    Span sp;
+    sp.pa = cxoff[oc0];
+    sp.pb = cxoff[oc0 + cols - 1] + cp.K;
+    sp.la = max(sp.pa, j.left - j.px0);
+    sp.lb = min(sp.pb, j.left + j.new_w - j.px0);
+    if (sp.live() < sp.width()) {
+        const int width = sp.width();
+        for (int i = threadIdx.x; i < CROP_RING * width; i += CROP_THREADS) {
+            const int px = sp.pa + i % width;
+            if (px < sp.la || px >= sp.lb) ring[i] = 0u;
+        }
+    }
     Columns<K> cs;
 #pragma unroll
     for (int q = 0; q < CROP_PASS; ++q) {
-        const int px = threadIdx.x + CROP_THREADS * q, x = min(max(j.px0 + px - j.left, 0), j.new_w - 1);
+        const int px = sp.la + min(int(threadIdx.x) + CROP_THREADS * q, max(sp.live() - 1, 0));
+        const int x = min(max(j.px0 + px - j.left, 0), j.new_w - 1);
         cs.x0[q] = ((const AS_GLOBAL int*)np.xoff)[x];
 #pragma unroll
         for (int k = 0; k < K; ++k) cs.w[q][k] = ((const AS_GLOBAL float*)np.xw)[x * K + k];
     }
-    const int ox = threadIdx.x;
-    const int ox0 = ((const AS_GLOBAL int*)cp.xoff)[ox];
+    const int ox = oc0 + min(int(threadIdx.x), cols - 1);
+    const int ox0 = ((const AS_GLOBAL int*)cp.xoff)[ox] - sp.pa;
     float ow[CROP_KMAX];
 #pragma unroll
     for (int k = 0; k < CROP_KMAX; ++k) ow[k] = k < cp.K ? ((const AS_GLOBAL float*)cp.xw)[ox * cp.K + k] : 0.0f;
     const auto ysi = (const AS_CONST int*)cp.ysi;
-    const RingSrc rs{ring, j.pw};
-    const bool words = (reinterpret_cast<uintptr_t>(out) & 3) == 0;
+    const RingSrc rs{ring, sp.width()};
+    const bool words = (reinterpret_cast<uintptr_t>(out) & 3) == 0, mine = int(threadIdx.x) < cols;
     uint8_t* d = out + 3 * CROP_W * oy0;
     int have = ysi[oy0 * cp.K];   // patch rows below this one are in the ring (or not needed)
     for (int oy = oy0; oy < oy1; ++oy, d += 3 * CROP_W) {
         const int need = ysi[oy * cp.K + cp.K - 1] + 1;
-        fill_rows<K, FIN>(j, np, src, cs, have, need, ring);
+        fill_rows<K, FIN>(j, np, src, cs, sp, have, need, ring);
         have = max(have, need);
         __syncthreads();
         const unsigned v = out_px_any(cp, rs, ox0, ow, oy);
-        if (words) {
+        if (words) {   // cols is a multiple of four: a lane quad is in or out
             const int i = ox & 3;
             const unsigned w = quad_word(v, i);
-            if (i < 3) *reinterpret_cast<unsigned*>(d + 3 * (ox - i) + 4 * i) = w;
-        } else {
+            if (mine && i < 3) *reinterpret_cast<unsigned*>(d + 3 * (ox - i) + 4 * i) = w;
+        } else if (mine) {
             d[3 * ox] = uint8_t(v);
             d[3 * ox + 1] = uint8_t(v >> 8);
             d[3 * ox + 2] = uint8_t(v >> 16);
@@ -357,50 +406,31 @@ __device__ __forceinline__ void crop_band(const JobDev& j, const PlanDev& np, co
     }
 }
 
-// Workgroup (band of output rows, crop) of five waves: per output row the canvas rows it adds (each thread its columns,
-// so a wave reads neighbouring pixels), then one output pixel per thread.  Reads the native pixels under a crop once (a
-// row or two more per band) and writes the crop; bound by the instructions of the row pass: a conversion, a product and
-// a sum per byte and tap.
-// Kernel time of 640 crops of 1920 x 1080 RGB frames 1.24 ms, of 80 crops of 1280 x 720 I420 frames 156 us; the calls 6.44 ->
-// 1.83 ms and 414 -> 237 us (two kernels, canvas patches through HBM, tap loops over byte loads before).
+// Workgroup (band of output rows and chunk of their columns, crop) of five waves: per output row the canvas rows it adds
+// (each thread its columns, so a wave reads neighbouring pixels), then one output pixel per thread.  Reads the native pixels
+// under a crop once (a row or two more per band) and writes the crop; bound by the instructions of the row pass for many
+// crops (a conversion, a product and a sum per byte and tap), by a workgroup's rows one after another for few.
+// Kernel time of 640 crops of 1920 x 1080 RGB frames 1.10 ms, of 80 crops of 1280 x 720 I420 frames 150 us; the calls 6.44 ->
+// 1.51 ms and 414 -> 197 us (two kernels, canvas patches through HBM, tap loops over byte loads before).
 template <bool I420, int V>
 __global__ void __launch_bounds__(CROP_THREADS)
-crop_kernel(const JobDev* __restrict__ jobs, const PlanDev* __restrict__ plans, uint8_t* __restrict__ out, Yuv yuv,
-            int band) {
+crop_kernel(const JobDev* __restrict__ jobs, const PlanDev* __restrict__ plans, uint8_t* __restrict__ out,
+            int band, int chunks) {
     extern __shared__ __attribute__((aligned(16))) unsigned ring[];
     constexpr int K = kVariants[V].K, FIN = kVariants[V].fin;
     const JobDev j = jobs[blockIdx.y];
-    const int oy0 = blockIdx.x * band, oy1 = min(CROP_H, oy0 + band);
+    const int cols = CROP_W / chunks, oc0 = int(blockIdx.x % chunks) * cols;
+    const int oy0 = int(blockIdx.x / chunks) * band, oy1 = min(CROP_H, oy0 + band);
     const PlanDev cp = plans[j.crop_plan], np = plans[j.canvas_plan];
     uint8_t* d = out + (long long)j.index * (CROP_W * CROP_H * 3);
     if constexpr (I420) {
         const I420Src src{global_bytes(j.frame), global_bytes(j.u), global_bytes(j.v), j.stride, j.u_stride, j.v_stride,
-                          np.sh, yuv};
-        crop_band<K, FIN>(j, np, cp, src, oy0, oy1, ring, d);
+                          np.sh};
+        crop_band<K, FIN>(j, np, cp, src, oy0, oy1, oc0, cols, ring, d);
     } else {
         const RgbSrc src{global_bytes(j.frame), j.stride, np.sh};
-        crop_band<K, FIN>(j, np, cp, src, oy0, oy1, ring, d);
+        crop_band<K, FIN>(j, np, cp, src, oy0, oy1, oc0, cols, ring, d);
     }
-}
-
-// 16-bit rounding of a 2^16-scaled coefficient with saturation (ffmpeg's round + av_clip_int16)
-int round_to_16(long long f) {
-    int r = int((f + (1 << 15)) >> 16);
-    if (r < -32768) r = -32768;
-    if (r > 32767) r = 32767;
-    return r;
-}
-Yuv yuv_coeffs() {
-    const long long cy = (65536LL * 255) / 219;   // contrast = saturation = 1 << 16 leave the table entries unscaled
-    Yuv k;
-    k.y_coeff = round_to_16(cy * (1 << 13));
-    k.vr = round_to_16(104597LL * (1 << 13));
-    k.ub = round_to_16(132201LL * (1 << 13));
-    k.ug = round_to_16(-25675LL * (1 << 13));
-    k.vg = round_to_16(-53279LL * (1 << 13));
-    k.y_off = round_to_16((16LL << 16) * (1 << 3));
-    k.uv_off = 0x0400;
-    return k;
 }
 
 // Plans uploaded once per geometry; the device plan table and the job tables grow as needed.  One call at a time.
@@ -434,7 +464,8 @@ public:
         JobDev* jd = static_cast<JobDev*>(jobs_host_);
         std::vector<JobDev> all(static_cast<size_t>(n));
         std::vector<int> kn(static_cast<size_t>(n));
-        int first[CROP_VARIANTS + 1] = {}, width[CROP_VARIANTS] = {};   // crops of each variant, widest patch
+        // per variant: crops, widest patch, widest resized frame
+        int first[CROP_VARIANTS + 1] = {}, patch_w[CROP_VARIANTS] = {}, frame_w[CROP_VARIANTS] = {};
         for (int i = 0; i < n; ++i) {
             const CropJob& j = jobs[i];
             const CanvasGeo& g = geo[size_t(i)];
@@ -452,7 +483,8 @@ public:
             const int k = crop_variant(np.K, np.fin, np.sw, i420);
             kn[size_t(i)] = k;
             ++first[k + 1];
-            width[k] = std::max(width[k], d.pw);
+            patch_w[k] = std::max(patch_w[k], d.pw);
+            frame_w[k] = std::max(frame_w[k], d.new_w);
         }
         for (int k = 1; k <= CROP_VARIANTS; ++k) first[k] += first[k - 1];
         int at[CROP_VARIANTS];
@@ -461,16 +493,14 @@ public:
         sync_plans();
         grow(jobs_dev_, jobs_bytes_, size_t(n) * sizeof(JobDev));
         CROP_CHECK(hipMemcpyAsync(jobs_dev_, jd, size_t(n) * sizeof(JobDev), hipMemcpyHostToDevice, s));
-        // bands per crop: enough workgroups for a few crops, 15 output rows each for many (a band recomputes a canvas
-        // row or two)
-        const int bands = std::max(12, std::min(60, (6144 + n - 1) / n)), band = (CROP_H + bands - 1) / bands;
-        static const Yuv yuv = yuv_coeffs();
         for (int k = 0; k < CROP_VARIANTS; ++k) {
             const int m = first[k + 1] - first[k];
             if (m == 0) continue;
-            const dim3 grid((CROP_H + band - 1) / band, m);
-            const size_t lds = size_t(CROP_RING) * width[k] * 4;
-            launch(std::make_integer_sequence<int, CROP_VARIANTS>(), i420, k, grid, lds, s, static_cast<const JobDev*>(jobs_dev_) + first[k], out, yuv, band);
+            const CropSplit split = crop_split(n, k, frame_w[k]);
+            const dim3 grid((CROP_H + split.band - 1) / split.band * split.chunks, m);
+            const size_t lds = size_t(CROP_RING) * ring_width(patch_w[k], CROP_W / split.chunks) * 4;
+            launch(std::make_integer_sequence<int, CROP_VARIANTS>(), i420, k, grid, lds, s,
+                   static_cast<const JobDev*>(jobs_dev_) + first[k], out, split);
             CROP_CHECK(hipGetLastError());
         }
         CROP_CHECK(hipStreamSynchronize(s));   // the job table is reused by the next call
@@ -487,17 +517,17 @@ private:
     size_t plans_bytes_ = 0, jobs_bytes_ = 0, jobs_host_bytes_ = 0;
 
     template <bool I420, int V>
-    void launch_variant(dim3 grid, size_t lds, hipStream_t s, const JobDev* j, uint8_t* out, const Yuv& yuv, int band) {
+    void launch_variant(dim3 grid, size_t lds, hipStream_t s, const JobDev* j, uint8_t* out, CropSplit split) {
         hipLaunchKernelGGL((crop_kernel<I420, V>), grid, dim3(CROP_THREADS), lds, s, j,
-                           static_cast<const PlanDev*>(plans_dev_), out, yuv, band);
+                           static_cast<const PlanDev*>(plans_dev_), out, split.band, split.chunks);
     }
     template <int... V>
     void launch(std::integer_sequence<int, V...>, bool i420, int v, dim3 grid, size_t lds, hipStream_t s, const JobDev* j,
-                uint8_t* out, const Yuv& yuv, int band) {
-        typedef void (CropEngine::*Go)(dim3, size_t, hipStream_t, const JobDev*, uint8_t*, const Yuv&, int);
+                uint8_t* out, CropSplit split) {
+        typedef void (CropEngine::*Go)(dim3, size_t, hipStream_t, const JobDev*, uint8_t*, CropSplit);
         static const Go go[2][CROP_VARIANTS] = {{&CropEngine::launch_variant<false, V>...},
                                                 {&CropEngine::launch_variant<true, V>...}};
-        (this->*go[i420][v])(grid, lds, s, j, out, yuv, band);
+        (this->*go[i420][v])(grid, lds, s, j, out, split);
     }
     static void grow(void*& p, size_t& have, size_t need) {
         if (need <= have) return;

@@ -9,7 +9,7 @@
 namespace shv {
 
 constexpr int CROP_W = 320, CROP_H = 180, COEF_BITS = 11, COEF_SCALE = 1 << COEF_BITS;
-constexpr int CROP_KMAX = 5;    // source pixels per axis of the unrolled kernels (scales up to 4)
+constexpr int CROP_KMAX = 5;    // canvas rows and columns per output pixel (scales up to 4)
 
 // how a column pass ends (rounding after a scale, 1 where there is none; the 2 x 2 blocks' and the linear resize's integer
 // forms have K = 2)
@@ -138,6 +138,22 @@ inline bool make_plan(int sw, int sh, int dw, int dh, int interpolation, PlanHos
     return true;
 }
 
+// ffmpeg's yuv2rgb coefficients for BT.601 limited range (contrast = saturation = 1 << 16, brightness 0), rounded to 16 bits
+// as av_clip_int16((x + 2^15) >> 16): Y 76309 (= 65536 * 255 / 219) and the inverse-table entries 104597 (V->R), 132201
+// (U->B), -25675 (U->G), -53279 (V->G), each times 2^13.  The reference works in 16 bits with saturation: (8 y - 128) Y >> 16,
+// (8 c - 1024) C >> 16 per chroma table, sums saturated.  No sum of these reaches 16 bits (8-bit operands), so only the last
+// one, to 8 bits, is left; as compile-time constants a term is one multiply-add and one shift.
+constexpr int yuv_round16(long long f) { return int((f + (1 << 15)) >> 16); }
+constexpr int YUV_Y = yuv_round16((65536LL * 255 / 219) * (1 << 13)), YUV_VR = yuv_round16(104597LL * (1 << 13)),
+              YUV_UB = yuv_round16(132201LL * (1 << 13)), YUV_UG = yuv_round16(-25675LL * (1 << 13)),
+              YUV_VG = yuv_round16(-53279LL * (1 << 13));
+constexpr int yuv_luma(int y) { return (y * (8 * YUV_Y) - 128 * YUV_Y) >> 16; }
+constexpr int yuv_term(int c, int coeff) { return (c * (8 * coeff) - 1024 * coeff) >> 16; }
+constexpr int yuv_red(int v) { return yuv_term(v, YUV_VR); }
+constexpr int yuv_green(int u, int v) { return yuv_term(u, YUV_UG) + yuv_term(v, YUV_VG); }
+constexpr int yuv_blue(int u) { return yuv_term(u, YUV_UB); }
+constexpr int yuv_sat8(int v) { return v < 0 ? 0 : (v > 255 ? 255 : v); }
+
 // canvas geometry of a w x h frame (geometry.cpp:77-88): scale min(720/h, 1280/w), centred, mode 0 copy /
 // 1 shrink (area) / 2 enlarge (linear)
 struct CanvasGeo {
@@ -158,8 +174,9 @@ inline bool canvas_geo(int w, int h, CanvasGeo& g) {
 // The launches take the crops of one canvas resize each: K taps and finish, or (0) whatever else.
 struct Variant { int K, fin; };
 constexpr Variant kVariants[] = {{0, FIN_SCALE}, {1, FIN_SCALE}, {2, FIN_SCALE}, {2, FIN_QUARTER}, {2, FIN_LINEAR},
-                                 {3, FIN_SCALE}, {4, FIN_SCALE}, {5, FIN_SCALE}};
-constexpr int CROP_VARIANTS = 8;
+                                 {3, FIN_SCALE}, {4, FIN_SCALE}, {5, FIN_SCALE}, {6, FIN_SCALE}, {7, FIN_SCALE},
+                                 {8, FIN_SCALE}};
+constexpr int CROP_VARIANTS = 11;
 
 // What an unrolled kernel reads of a source row for the K pixels from a column on: whole words, so up to three bytes past
 // them.  Those lie in the next row, which is there: rows of the plane's last pixel row (I420: last chroma row) are read byte
@@ -173,5 +190,23 @@ inline int crop_variant(int K, int fin, int sw, bool i420) {   // of a plan over
     while (k > 0 && !(K == kVariants[k].K && fin == kVariants[k].fin)) --k;
     return k;
 }
+
+// How the crops of one kernel (variant) are split in a call of n, frames resized to new_w columns: bands of `band` output
+// rows, and 1, 2 or 4 chunks of their columns.  A band or chunk computes a canvas row or a few columns again, but a workgroup
+// walks its rows one after another: few crops want many short ones.  Calls in us: one crop of a 1920 x 1080 frame RGB 36 in
+// bands of 3 rows, 25 in 1 row x 2 chunks (I420 56, 27), 4 RGB 40 in 3 rows, 34 in 1, 8 RGB 51 in 3, 46 in 2, 50 in 1, 40 RGB
+// 116 in 3, 136 in 1.  7680 x 4320 I420 (6 taps): 4 crops 217 in 1 row, 185 in 3 x 2 chunks, 10 crops 524 in 3, 449 in 3 x 2.
+// More than 8 taps: one crop of 9000 x 5000 RGB 293 in 1 x 2, 225 in 1 x 4, 20 of 20000 x 100 1,606 in 3, 709 in 1 x 4, but 20
+// of 100 x 20000 (4 live columns) 386 in 3, 1,638 in 1 x 4.
+struct CropSplit { int band, chunks; };
+inline CropSplit crop_split(int n, int variant, int new_w) {
+    if (variant == 0 && new_w >= CROP_W) return {1, 4};   // 81 taps a pixel and more: as many threads as there are pixels
+    if (kVariants[variant].K > CROP_KMAX && n > 1 && n <= 16) return {3, 2};
+    const int bands = n <= 4 ? 180 : n <= 8 ? 90 : std::max(12, std::min(60, (6144 + n - 1) / n));
+    return {(CROP_H + bands - 1) / bands, n <= 2 ? 2 : 1};
+}
+// Most patch columns under `cols` output columns of a patch pw wide: their cells and a pixel on either side, or the K
+// pixels to which the last columns' taps are pulled back.
+inline int ring_width(int pw, int cols) { return std::min(pw, (cols * pw + CROP_W - 1) / CROP_W + CROP_KMAX + 1); }
 
 }  // namespace shv

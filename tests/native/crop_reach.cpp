@@ -34,8 +34,22 @@ static long long reach(int w, int h, bool i420) {
     return worst;
 }
 
+static int sat16(int v) { return v < -32768 ? -32768 : (v > 32767 ? 32767 : v); }
+
 int main() {
     int frames = 0, bad = 0;
+    // every I420 pixel against the 16-bit arithmetic with its saturations
+    const int yc = 9539, vr = 13075, ub = 16525, ug = -3209, vg = -6660;
+    for (int y = 0; y < 256; ++y)
+        for (int u = 0; u < 256; ++u)
+            for (int v = 0; v < 256; ++v) {
+                const int yy = (int(short((y << 3) - 128)) * yc) >> 16, up = sat16((u << 3) - 1024), vp = sat16((v << 3) - 1024);
+                const int r = yuv_sat8(sat16(yy + ((vp * vr) >> 16))), b = yuv_sat8(sat16(yy + ((up * ub) >> 16)));
+                const int g = yuv_sat8(sat16(yy + sat16(((up * ug) >> 16) + ((vp * vg) >> 16))));
+                const int l = yuv_luma(y);
+                if (yuv_sat8(l + yuv_red(v)) != r || yuv_sat8(l + yuv_green(u, v)) != g || yuv_sat8(l + yuv_blue(u)) != b) ++bad;
+            }
+    if (bad) std::printf("%d I420 pixels differ\n", bad);
     const auto check = [&](int w, int h) {
         for (int i420 = 0; i420 < 2; ++i420, ++frames) {
             const long long r = reach(w, h, i420);
@@ -47,6 +61,21 @@ int main() {
     for (int h = 1; h <= 12; ++h)
         for (int w = 25; w <= 6000; w += 131) check(w, h);
     for (int s = 1; s <= 40; ++s) check(160 * s, 90 * s), check(90 * s, 160 * s), check(160 * s + 1, 90 * s + 1);
+    // the LDS ring holds the patch columns of every chunk of output columns
+    for (int w4 = 80; w4 <= 320; ++w4)
+        for (int chunks = 1; chunks <= 4; chunks *= 2) {
+            const int pw = 4 * w4, cols = CROP_W / chunks;
+            PlanHost p;
+            if (!make_plan(pw, 4 * 45, CROP_W, CROP_H, 3, p) || p.K > CROP_KMAX) {
+                ++bad;
+                continue;
+            }
+            for (int c = 0; c < CROP_W; c += cols) {
+                const int need = p.xoff[size_t(c + cols - 1)] + p.K - p.xoff[size_t(c)];
+                if (need > ring_width(pw, cols) && ++bad <= 20)
+                    std::printf("patch %d: %d columns, room for %d\n", pw, need, ring_width(pw, cols));
+            }
+        }
     std::printf("%d frames, %d out of range\n", frames, bad);
     return bad ? 1 : 0;
 }

@@ -2000,14 +2000,22 @@ bool use_gemv_f32(const GemmArgs& p) {
 
 void gemm_f32_mfma(const GemmArgs& p, hipStream_t s) {
     check_args(p, false);
-    if (!gemm_f32_mc_ok(p))
+    if (!v4_f32_ok(p))
         throw std::runtime_error("gemm_f32_mfma: K, lda, ldw, ld_scale must be multiples of 4 and A, W, scale "
                                  "16-byte aligned (K=" + std::to_string(p.K) + ")");
     if (p.swiglu && p.N % 32) throw std::runtime_error("gemm_f32_mfma: swiglu needs N % 32 == 0");
-    gemm_f32_mc(p, p.swiglu ? 2 : 0, s);
+    if (gemm_f32_mc_ok(p)) {
+        gemm_f32_mc(p, p.swiglu ? 2 : 0, s);
+        return;
+    }
+    // rows past the matrix-core kernels' 32-bit offsets: the VALU kernel's, the same sequence (its SwiGLU takes other panels)
+    if (p.swiglu) throw std::runtime_error("gemm_f32_mfma: leading dimension too large");
+    launch_tiled_f32(p, s);
 }
 
-std::string gemm_f32_mfma_kernel_name(const GemmArgs& p) { return gemm_f32_mc_kernel(p, p.swiglu ? 2 : 0); }
+std::string gemm_f32_mfma_kernel_name(const GemmArgs& p) {
+    return gemm_f32_mc_ok(p) ? gemm_f32_mc_kernel(p, p.swiglu ? 2 : 0) : "gemm_f32_v4_kernel";
+}
 
 void gemm_f32(const GemmArgs& p, hipStream_t s) { gemm_f32_variant(p, s, 0); }
 

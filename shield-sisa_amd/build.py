@@ -27,7 +27,7 @@ OBJ = PKG / "_obj"
 LIB = PKG / "lib"
 INCLUDE = PKG.parent / "include"
 
-NUMERIC_SOURCES = ["dev_common.hpp", "mfma.hpp", "kernels.hpp", "gemm_epi.hpp", "gemm_reach.hpp", "gemm.hip",
+NUMERIC_SOURCES = ["dev_common.hpp", "silu_near.hpp", "mfma.hpp", "kernels.hpp", "gemm_epi.hpp", "gemm_reach.hpp", "gemm.hip",
                    "gemm_f32.hpp", "gemm_f32.hip", "cnn.hip", "expdw.hip", "fused.hip", "strip.hip", "seq.hip",
                    "engine.hpp", "engine.hip", "stack.hpp", "audio.hpp", "audio.hip", "afront.hip",
                    "host_model.hpp", "host_model.cpp"]

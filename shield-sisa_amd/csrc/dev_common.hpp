@@ -6,6 +6,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "silu_near.hpp"
+
 namespace shv {
 
 typedef _Float16 f16;
@@ -48,24 +50,6 @@ __device__ __forceinline__ float silu(float x) { return x / (1.0f + cephes_exp(0
 // Limits: x -> -inf gives -0, x -> +inf gives x, NaN stays NaN.
 __device__ __forceinline__ float silu_fast(float x) {
     return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.44269504088896341f));
-}
-// SiLU in 16 instructions (silu() and the libm form take 35 to 45): exp(-x) = 2^n 2^f with the hardware exp2 of the
-// fraction, then x / (1 + exp(-x)) by the hardware reciprocal and one residual step against 1 + exp(-x) unrounded.
-// Against 64 bits over 4 M normal x of scale 0.01 to 40 its relative error is 0.4e-8 to 2.9e-8 (silu() 0.6e-8 to 4.4e-8,
-// the libm form the same), its mean 0.22 to 0.29 ulp (0.25 to 0.42).  Limits: the exponent's argument is clamped where
-// 2^n leaves the normal numbers (below -87.3 the result is -0, as the libm form's below -88.7); div_fixup gives an
-// infinite or NaN x its IEEE quotient.
-__device__ __forceinline__ float silu_near(float x) {
-    constexpr float MAGIC = 12582912.0f;   // 1.5 * 2^23: its sum with |y| < 2^22 holds rint(y) in the low bits
-    const float c = __builtin_amdgcn_fmed3f(x, -87.4f, 87.0f);
-    const float m = __builtin_fmaf(c, -1.44269504088896341f, MAGIC), n = m - MAGIC;
-    float f = __builtin_fmaf(c, -1.44269504088896341f, -n);
-    f = __builtin_fmaf(c, -1.92596299e-8f, f);
-    const float e = __int_as_float(__float_as_int(__builtin_amdgcn_exp2f(f)) + (__float_as_int(m) << 23));
-    const float d = 1.0f + e, dl = e - (d - 1.0f), r = __builtin_amdgcn_rcpf(d);   // d + dl is 1 + e exactly
-    float q = x * r;
-    q = __builtin_fmaf(__builtin_fmaf(-dl, q, __builtin_fmaf(-d, q, x)), r, q);
-    return __builtin_amdgcn_div_fixupf(q, d, x);
 }
 __device__ __forceinline__ float relu(float x) { return x > 0.0f ? x : 0.0f; }
 

@@ -1520,10 +1520,22 @@ __global__ void __launch_bounds__(256, 2) gemm_wide_kernel(GemmArgs p) {
 }
 // groups of four tiles (256-byte row pieces) where the registers allow, else two (fp16 K <= 192, bf16 K <= 128)
 template <typename T, int KS> void launch_wide_ks(const GemmArgs& p, hipStream_t s) {
-    constexpr int GR = (Split<T>::P == 2 ? KS <= 6 : KS <= 4) ? 4 : 2;
+    constexpr int KS4 = Split<T>::P == 2 ? 6 : 4;   // most K steps whose group of four tiles fits the registers, all but 18
+    constexpr int GR = KS <= KS4 ? 4 : 2;
     const size_t lds = size_t(Split<T>::P) * WD_ROWS * (KS * 32 + WD_PAD) * sizeof(T) +
                        size_t(4) * 16 * WD_SLD * sizeof(float);
-    hipLaunchKernelGGL((gemm_wide_kernel<T, KS, GR>), dim3(cdiv(p.M, WD_ROWS)), dim3(256), lds, s, p);
+    const dim3 grid(cdiv(p.M, WD_ROWS));
+    // Those 18 spilled ones cost more than the longer stores of four tiles give, except where groups of two leave the four
+    // waves uneven, 12 tiles or fewer; four / two in us, fp16 K 192: 53,802 rows N 480 74.5 / 66.3, N 960 127 / 115, 200,000
+    // rows N 180 118 / 129; bf16 K 112: 53,802 rows N 240 35.5 / 32.7, N 320 50.0 / 41.8, K 128 200,000 rows N 180 111 / 124
+    // (tile by tile, before the pairs: 70.0, 120, 132, 34.5, 48.8, 120).
+    if constexpr (KS == KS4) {
+        if (p.N > 12 * 16) {
+            hipLaunchKernelGGL((gemm_wide_kernel<T, KS, 2>), grid, dim3(256), lds, s, p);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((gemm_wide_kernel<T, KS, GR>), grid, dim3(256), lds, s, p);
 }
 bool wide_ok(const GemmArgs& p) {
     const auto al16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };

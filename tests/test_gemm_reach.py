@@ -24,3 +24,10 @@ def test_weight_reads_stay_in_their_row(tmp_path):
 @pytest.mark.parametrize("mode", ["fp16", "bf16"])
 def test_short_rows(shv, mode, M, N, K):
     wide.test_wide_gemm_equals_direct(shv, mode, M, N, K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N", [192, 196, 324, 960])   # 12 column tiles in groups of four, 13, 21 (odd) and 60 in groups of two
+@pytest.mark.parametrize("mode,K", [("fp16", 184), ("fp16", 192), ("bf16", 104), ("bf16", 128)])
+def test_groups_of_two_or_four_tiles(shv, mode, N, K):
+    wide.test_wide_gemm_equals_direct(shv, mode, 2113, N, K)

@@ -2002,11 +2002,19 @@ void launch_narrow_f32(const GemmArgs& p, hipStream_t s) {
         throw std::runtime_error("gemm_f32: no narrow kernel for K=" + std::to_string(p.K) + " N=" + std::to_string(p.N) +
                                  " with these leading dimensions / alignments");
 }
-// Few rows stay on the GEMV, which reads W once whatever its alignment (one row: 6.1-6.2 us against 7.0-7.2 of the
-// matrix-core kernels; 20 rows 7.3-9.5 against 6.3-7.4, 128 rows 22-56 against 7-9); without the matrix cores' alignment
-// it serves every M it takes.
+// The GEMV reads W once whatever its alignment, and keeps few outputs: up to 4 rows (one row: 6.1-6.2 us against 7.0-7.2 of
+// the matrix-core kernels), and few rows times columns, where its waves (64 lanes of K blocks) fit the device once.  GEMV /
+// matrix cores in us, K a multiple of 64: 16 x 16 x 960 4.1 / 6.4, 16 x 16 x 2048 4.4 / 10.3, 16 x 100 x 1024 5.1 / 6.8, 25 x
+// 100 x 1024 (2,500 outputs) 6.1 / 7.0, 16 x 200 x 1024 (3,200) 6.9 / 6.9, 25 x 200 x 1024 7.8 / 7.0, 40 x 100 x 1024 (4,000,
+// two rows a workgroup past 32) 6.7 / 7.0, 64 x 69 x 1024 8.0 / 7.0, 64 x 40 x 512 5.4 / 5.2, 16 x 200 x 2048 9.8 / 10.5; with a shorter last block: 25 x 40 x 1756 7.8 / 8.3, 16 x 69 x 1756 8.4 / 8.3, 40 x 16 x 1756
+// 9.9 / 8.3, 5 x 16 x 1028 7.4 / 6.6.  Past those 20 rows take 7.3-9.5 / 6.3-7.4, 128 rows 22-56 / 7-9.  Without the matrix
+// cores' alignment it serves every M it takes.
 bool use_gemv_f32(const GemmArgs& p) {
-    return p.M <= (gemm_f32_mc_ok(p) ? 4 : GV_MAXM) && cdiv(p.K, F32_BK) <= 32;
+    if (cdiv(p.K, F32_BK) > 32) return false;
+    if (p.M <= 4 || !gemm_f32_mc_ok(p)) return p.M <= GV_MAXM;
+    const long long outputs = (long long)p.M * p.N;
+    if (p.K % F32_BK == 0) return outputs <= (p.M > 32 || p.K >= 1536 ? 4000 : 2560) && p.M <= (p.K >= 768 ? 64 : 32);
+    return outputs <= 1024 && p.M <= 32 && p.K >= 1400;
 }
 }  // namespace
 

@@ -493,7 +493,8 @@ public:
         sync_plans();
         grow(jobs_dev_, jobs_bytes_, size_t(n) * sizeof(JobDev));
         CROP_CHECK(hipMemcpyAsync(jobs_dev_, jd, size_t(n) * sizeof(JobDev), hipMemcpyHostToDevice, s));
-        for (int k = 0; k < CROP_VARIANTS; ++k) {
+        hipError_t launched = hipSuccess;
+        for (int k = 0; k < CROP_VARIANTS && launched == hipSuccess; ++k) {
             const int m = first[k + 1] - first[k];
             if (m == 0) continue;
             const CropSplit split = crop_split(n, k, frame_w[k]);
@@ -501,9 +502,11 @@ public:
             const size_t lds = size_t(CROP_RING) * ring_width(patch_w[k], CROP_W / split.chunks) * 4;
             launch(std::make_integer_sequence<int, CROP_VARIANTS>(), i420, k, grid, lds, s,
                    static_cast<const JobDev*>(jobs_dev_) + first[k], out, split);
-            CROP_CHECK(hipGetLastError());
+            launched = hipGetLastError();
         }
-        CROP_CHECK(hipStreamSynchronize(s));   // the job table is reused by the next call
+        const hipError_t done = hipStreamSynchronize(s);   // after a failed launch too: the next call reuses the job tables
+        CROP_CHECK(launched);
+        CROP_CHECK(done);
     }
 
 private:

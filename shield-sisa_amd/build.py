@@ -27,7 +27,7 @@ OBJ = PKG / "_obj"
 LIB = PKG / "lib"
 INCLUDE = PKG.parent / "include"
 
-NUMERIC_SOURCES = ["dev_common.hpp", "silu_near.hpp", "mfma.hpp", "kernels.hpp", "gemm_epi.hpp", "gemm_reach.hpp", "gemm.hip",
+NUMERIC_SOURCES = ["dev_common.hpp", "silu_near.hpp", "mfma.hpp", "kernels.hpp", "gemm_reach.hpp", "gemm.hip",
                    "gemm_f32.hpp", "gemm_f32.hip", "cnn.hip", "expdw.hip", "fused.hip", "strip.hip", "seq.hip",
                    "engine.hpp", "engine.hip", "stack.hpp", "audio.hpp", "audio.hip", "afront.hip",
                    "host_model.hpp", "host_model.cpp"]
@@ -47,9 +47,11 @@ DEVICE_FLAGS = ["--offload-arch=" + ARCH, "-Xclang", "-target-feature", "-Xclang
 # MFMA accumulators in ordinary VGPRs instead of AGPRs (the unified register file holds them either way; the AGPR
 # form adds v_accvgpr moves around every accumulation chain and costs registers).  Only for sources where no inline
 # asm reads an MFMA result: the compiler inserts the MFMA-to-VALU wait states for its own instructions but not for
-# an asm operand, and an empty asm is counted as one wait state.  In these two files every asm operand is a loaded
-# value or a VALU result; tests/test_mfma_asm_hazard.py checks that on the built code objects (no inline-asm DPP
-# instruction reads a VGPR that an MFMA write can reach).
+# an asm operand, and an empty asm is counted as one wait state.  In these files every operand of an asm instruction is a
+# loaded value or a VALU result; tests/test_mfma_asm_hazard.py checks that on the built code objects (no inline-asm DPP
+# instruction reads a VGPR that an MFMA write can reach).  gemm.hip's scheduling fence, an empty asm, does take the wide
+# kernel's accumulators: their first reader behind it (the group's epilogue) is more than 50 instructions away, an MFMA's
+# result 11 wait states.
 VGPR_FORM_SOURCES = {"strip.hip", "gemm.hip", "gemm_f32.hip", "expdw.hip"}
 VGPR_FORM_FLAGS = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 

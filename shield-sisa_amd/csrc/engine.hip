@@ -462,7 +462,7 @@ private:
         dump_f32(dump_dir_, name, dev, n, s);
     }
 
-    // GEMM in this engine's flavour, and the exact fp32 VALU kernel for the fp32-only layers
+    // GEMM in this engine's flavour, and the exact fp32 one for the fp32-only layers
     void gemm(const char* role, const GemmArgs& p, const DevW& w, hipStream_t s) {
         GemmRunner<G>{*this, cpu_order_}.gemm(role, p, w, s);
     }
@@ -845,7 +845,7 @@ void PwGemm::run(const float* A, long long M, const float* bias, int act, float*
     SHV_HIP_CHECK(hipGetLastError());
 }
 
-// One engine flavour per precision: the exact VALU tier, or the split-operand MFMA tiers with two (fp16) or three
+// One engine flavour per precision: the exact fp32 tier, or the split-operand MFMA tiers with two (fp16) or three
 // (bf16) operand parts.
 template <typename G> std::unique_ptr<Engine> engine_of(const HostModel& hm, Precision p, const EngineConfig& cfg) {
     return std::unique_ptr<Engine>(new EngineT<G>(hm, p, cfg));

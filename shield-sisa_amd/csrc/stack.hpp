@@ -183,7 +183,7 @@ template <typename U> void dump_f32(const std::string& dir, const char* name, co
 template <typename G> struct GemmRunner {
     static constexpr bool kF32 = std::is_same<G, float>::value;
     Profiler& pf;
-    bool cpu_order = false;   // fp32 tier: SwiGLU weights in the VALU kernels' gate / up pairs
+    bool cpu_order = false;   // fp32 tier: SwiGLU weights in adjacent gate / up pairs
     std::string family(const char* role, const GemmArgs& p, bool f32) const {
         if (!pf.profiling()) return std::string();
         if constexpr (!kF32) {
@@ -227,7 +227,7 @@ struct SeqSpec {
 
 // The sequence stages on the device: weights, activations for max_windows windows, and the forward from the
 // windows' token rows (WindowInput) to one logit per window.  Activations are fp32 in HBM in every tier;
-// G picks the GEMM arithmetic (float: exact VALU order; f16 / bf16: split-operand MFMA with the GEMM A operands
+// G picks the GEMM arithmetic (float: the exact fp32 order; f16 / bf16: split-operand MFMA with the GEMM A operands
 // written pre-split by their producers).
 template <typename G> class SeqStack {
     static constexpr bool kF32 = std::is_same<G, float>::value;
@@ -239,7 +239,7 @@ public:
              DevMem& amem)
         : spec_(spec) {
         cpu_order_ = kF32 && f32_cpu_order_requested();
-        const int swiglu_perm = cpu_order_ ? 1 : 2;   // VALU pairs (2j, 2j + 1) or MFMA 16-row panels
+        const int swiglu_perm = cpu_order_ ? 1 : 2;   // pairs (2j, 2j + 1) or 16-row panels
         for (int g = 0; g < 2; ++g) {
             const GdnHost& gh = gdn[g];
             Gdn& d = gdn_[g];

@@ -1,7 +1,8 @@
 // The bytes that the crop kernel's word loads touch, worked out from its own plans, choice of kernel and word counts
 // (shield-sisa_amd/csrc/crop_plan.hpp): over frames of any size, stored with the tightest strides and nothing after the last
 // pixel, no load may end past its plane.  A row of the plane's last pixel row (I420: last chroma row) is read byte by byte,
-// and so is everything in variant 0.
+// and so is everything in variant 0.  Beside it: the LDS ring holds a chunk's patch columns, and the I420 conversion equals
+// its 16-bit form.
 #include <cstdio>
 
 #include "../../shield-sisa_amd/csrc/crop_plan.hpp"

@@ -160,7 +160,7 @@ int shv_hip_set_dump_dir(shv_hip_model* m, const char* dir);
  * 4 the fp32 matrix cores (CPU order, k % 4 == 0), 5 narrow (CPU order; the (k, n) shapes of blocks 1-6 only: 16x16, 16x64,
  * 64x24, 24x72, 72x24, 72x40, 40x120, 120x40), 6 column chunks (CPU order, k <= 1024, k % 4 == 0); fp16 / bf16:
  * 1 small-M, 2..6 direct with
- * 1..5 column tiles per wave, 7 LDS-staged, 8 streaming (n <= 160).  Returns 0, or -1 + last_error.  Asynchronous on
+ * 1..5 column tiles per wave, 7 LDS-staged, 8 streaming (n <= 160), 9 wide (n % 4 == 0, k <= 256, bf16 <= 192).  Returns 0, or -1 + last_error.  Asynchronous on
  * `stream` except fp32 variant 3. */
 typedef struct shv_hip_gemm shv_hip_gemm;
 shv_hip_gemm* shv_hip_gemm_create(const char* mode, int n, int k, const float* d_w, void* stream);
@@ -198,10 +198,9 @@ int shv_hip_native_crops_i420(const shv_hip_i420_image* frames, const shv_hip_re
  * the reference runs its delta_kernel only inside classify, engine/cuda/seq.cu:106-195).  Per window 321 rows; rows
  * = n_windows * 321: q, k [rows][384] (6 heads x 64, l2-normalised; q scaled), v, o [rows][768] (6 heads x 128),
  * decay, beta [rows][8] (head h in column h).  Per (window, head): S_0 = 0, S_t = a_t S_{t-1} + k_t u_t^T,
- * u_t = b_t (v_t - a_t S_{t-1}^T k_t), o_t = S_t^T q_t.  variant 0: the tier's own kernel (fp32: token by token
- * with each value column's keys split over lane groups, or in the reference's order when SHV_HIP_F32_CPU_ORDER=1;
- * fp16 / bf16: the chunked scan), 1: token by token (fp32: the reference's order; fp16 / bf16: key split),
- * 2: chunked (fp16 / bf16), 3: key split (every tier).  Synchronous for the chunked scan (it allocates a work buffer
+ * u_t = b_t (v_t - a_t S_{t-1}^T k_t), o_t = S_t^T q_t.  variant 0: the tier's own kernel (the chunked scan; fp32
+ * token by token in the reference's order when SHV_HIP_F32_CPU_ORDER=1), 1: token by token (fp32: the reference's
+ * order; fp16 / bf16: key split), 2: chunked (every tier), 3: key split (every tier).  Synchronous for the chunked scan (it allocates a work buffer
  * per call).  Returns 0, or -1 + last_error. */
 int shv_hip_delta_rule(const char* mode, const float* d_q, const float* d_k, const float* d_v, const float* d_decay,
                        const float* d_beta, int n_windows, float* d_o, int variant, void* stream);

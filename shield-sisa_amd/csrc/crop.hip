@@ -409,7 +409,8 @@ __device__ __forceinline__ void crop_band(const JobDev& j, const PlanDev& np, co
 // Workgroup (band of output rows and chunk of their columns, crop) of five waves: per output row the canvas rows it adds
 // (each thread its columns, so a wave reads neighbouring pixels), then one output pixel per thread.  Reads the native pixels
 // under a crop once (a row or two more per band) and writes the crop; bound by the instructions of the row pass for many
-// crops (a conversion, a product and a sum per byte and tap), by a workgroup's rows one after another for few.
+// crops (a conversion, a product and a sum per byte and tap; VALU 60% busy at 640 crops, four waves a SIMD, 2.1 TB/s), by a
+// workgroup's rows one after another for few.
 // Kernel time of 640 crops of 1920 x 1080 RGB frames 1.10 ms, of 80 crops of 1280 x 720 I420 frames 150 us; the calls 6.44 ->
 // 1.51 ms and 414 -> 197 us (two kernels, canvas patches through HBM, tap loops over byte loads before).
 template <bool I420, int V>

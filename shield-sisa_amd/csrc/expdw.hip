@@ -13,12 +13,13 @@
 // theirs; SHIELD-A: sum of products over (kf, kt), BatchNorm, SiLU as silu_near()).  Few images: the chunks are dealt
 // over blockIdx.y too.
 //
-// Bound: fp32 by the matrix cores and the vector units together (an fp32 MFMA blocks its SIMD's vector instructions); the
-// half types by vector instructions (SiLU, depthwise) and the D stores.  So SiLU is the 16-instruction form, and the next
-// chunk's expand weights are read before the depthwise's stores (a load behind a store waits for it).  Against the
-// expand GEMM and the depthwise kernel apart, which wrote and read E: 32 clips in fp32 11.30 -> 9.36 ms, one clip
-// 1214 -> 1142 us; 128 SHIELD-A windows fp16 13.9 -> 11.5 ms, 5 windows fp32 967 -> 939 us.  SHIELD-A's first block also
-// computes its input, the stem, from the log-mel tile in LDS, once per band in the fragments' own layout: a stem kernel
+// Bound (MFMA / VALU busy by counters): SHIELD-A's early blocks by vector instructions, SiLU and depthwise (A0 6 / 96%, A1 7
+// / 68%), B2-B4 by them and memory (17-30 / 30-36% at 1.8-2.7 TB/s), the late blocks of both by a workgroup's waits between
+// its barriers, with one and a half waves a SIMD (B13 23 / 19%, B14 14 / 18%, A5 6 / 27%, A7 6 / 22%).  So SiLU is the
+// 16-instruction form, and the next chunk's expand weights are read before the depthwise's stores (a load behind a store
+// waits for it).  Against the expand GEMM and the depthwise kernel apart, which wrote and read E: 32 clips in fp32 11.30 ->
+// 9.36 ms, one clip 1214 -> 1142 us; 128 SHIELD-A windows fp16 13.9 -> 11.5 ms, 5 windows fp32 967 -> 939 us.  SHIELD-A's
+// first block also computes its input, the stem, from the log-mel tile in LDS, once per band in the fragments' own layout: a stem kernel
 // wrote 163 MB per 16 windows in 113 us (each thread loaded its 72 weights) and the block took 105 us; together 125 us,
 // 128 windows fp16 11.5 -> 10.6 ms, 5 windows fp32 939 -> 907 us.
 #include "dev_common.hpp"

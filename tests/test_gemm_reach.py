@@ -1,6 +1,6 @@
 """The wide pointwise GEMM reads no weight outside its row: on the CPU the lane offsets that the kernel compiles
 (tests/native/gemm_reach.cpp), on the GPU the shortest rows (K 8 to 24, fewer than a K step of 32) and the automatic choice
-for them, bitwise against the direct kernel."""
+for them, bitwise against the direct kernel.  Beside it, both sides of its groups of two or four column tiles."""
 import subprocess
 from pathlib import Path
 
